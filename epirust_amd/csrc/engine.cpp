@@ -451,10 +451,11 @@ int capture_day_graph(epi_sim* s) {
   return EPI_OK;
 }
 
+// The simulations' states after the last enqueued hour, from the pinned copies its epilogue
+// wrote: no copy, only the wait for the stream.
 int fetch_states(epi_sim* s) {
-  HIP_TRY(hipMemcpyAsync(s->state_h.data(), s->v.state, s->n_sims * sizeof(SimState), hipMemcpyDeviceToHost,
-                         s->stream));
   HIP_TRY(hipStreamSynchronize(s->stream));
+  std::memcpy(s->state_h.data(), s->pinned_state, s->n_sims * sizeof(SimState));
   return EPI_OK;
 }
 

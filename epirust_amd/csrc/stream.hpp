@@ -17,12 +17,12 @@ struct StreamArgs {
   uint32_t n;
   const SimState* state;  // records are written only if state->hour == hour
   uint32_t hour;
-  unsigned long long* block_off;  // stream_blocks(n) entries of scratch
+  unsigned long long* block_off;  // stream_blocks(n) entries of scratch: record lengths
   unsigned long long* total;      // bytes written this hour
   char* text;                     // >= n * max_record_bytes(...) bytes
 };
 
-// Agents the no-allocation formatter handles: its per-block offsets live in a static
+// Agents the no-allocation formatter handles: its record lengths live in a static
 // device array of kNoAllocMaxBlocks entries (8 bytes each).
 constexpr uint32_t kNoAllocMaxBlocks = 65536;
 constexpr uint32_t kNoAllocMaxAgents = kNoAllocMaxBlocks * 256u;
