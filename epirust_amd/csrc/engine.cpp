@@ -102,6 +102,16 @@ struct StateSink {
 
 }  // namespace
 
+// Groups of hours of a day that can run as one launch each:
+//   DAY_NIGHT   hours of day 1..6, when no vaccination falls at 1..5 (the only sweep pending in
+//               the night is then hour of day 0's) and no simulation's last hour at 1..6 (none
+//               stops inside the launch, whose agent blocks read the stop flag while its
+//               epilogues run; in a batch a day may hold a shorter run's last hour);
+//   DAY_QUIET   the epilogues of hours of day 3..6, when no vaccination falls at 2..5.
+// Lockdown, unlock and hospital decisions fall on hours of day 0 only; unlock needs h =
+// zero_infection_hour + 504, and that stays 0 in standalone mode.
+enum : uint8_t { DAY_NIGHT = 1, DAY_QUIET = 2, DAY_VARIANTS = 4 };
+
 struct epi_sim {
   std::vector<Config> cfg;
   std::vector<uint64_t> seed;
@@ -131,17 +141,12 @@ struct epi_sim {
   TileRef* d_tiles = nullptr;          // layout move tiles of every simulation
   uint32_t n_tiles = 0;
   uint64_t cap_blocks = 0, cap_office_blocks = 0;  // entries of the two device tables
-  // Day graphs run hours of day 3..6 as one epilogue-only launch: no simulation has a
-  // vaccination at an hour of day 2..5, so no sweep is pending at 3..6.
-  bool quiet_hours = false;
-  // ... and hours of day 1..6 as one launch when none has one at 1..5 either, and no
-  // simulation's last hour falls at 1..6 (a batch's day graph may hold a shorter run's
-  // last hour): then no simulation stops inside the launch, whose agent blocks read the
-  // stop flag while its epilogues run.
-  bool night = false;
+  // Per day (hours 24 d + 1 .. 24 d + 24), the groups of its hours that run as one launch
+  // (DAY_*): those inside which no sweep is decided and no simulation reaches its last hour.
+  std::vector<uint8_t> day_flags;
   SimDesc* d_desc = nullptr;
   hipStream_t stream = nullptr;
-  hipGraphExec_t day_graph = nullptr;
+  hipGraphExec_t day_graph[DAY_VARIANTS] = {};  // by the day's flags
   hipEvent_t poll_event[2] = {nullptr, nullptr};
   hipEvent_t loop_event[2] = {nullptr, nullptr};  // around the hour loop of one step call
   double last_loop_ms = 0.0;                      // device time of the last step call's hours
@@ -164,7 +169,8 @@ struct epi_sim {
   std::unique_ptr<StateSink> sink;  // citizen-state stream, single-simulation handles only
 
   ~epi_sim() {
-    if (day_graph) (void)hipGraphExecDestroy(day_graph);
+    for (hipGraphExec_t g : day_graph)
+      if (g) (void)hipGraphExecDestroy(g);
     for (auto& e : poll_event)
       if (e) (void)hipEventDestroy(e);
     for (auto& e : loop_event)
@@ -219,6 +225,15 @@ int validate(const Config& c) {
 // (workgroup w to XCD w % 8), in increasing order within each, and each XCD has its own L2.
 constexpr uint32_t kXcds = 8;
 
+AgentBlock office_block(uint64_t agent_off, uint32_t sim, uint32_t first, uint32_t count, uint32_t j_lo, uint32_t j_hi,
+                        uint32_t whole) {
+  AgentBlock e{agent_off, sim, first, count, {}};
+  e.j_lo = j_lo;
+  e.j_hi = j_hi;
+  e.whole = whole;
+  return e;
+}
+
 int build_launch_tables(epi_sim* s) {
   const uint32_t B = s->shape.block;
   s->agent_blocks.clear();
@@ -246,7 +261,9 @@ int build_launch_tables(epi_sim* s) {
     }
     for (uint32_t j = 0; j < nb; ++j) {
       const uint32_t first = sorted[start[j % kXcds] + j / kXcds] * B;
-      s->agent_blocks.push_back(AgentBlock{i, first, std::min(B, n - first), 1, 0, 1, 0, 0});
+      AgentBlock e{s->desc[i].agent_off, i, first, std::min(B, n - first), {}};
+      e.houses = s->desc[i].fd_houses;
+      s->agent_blocks.push_back(e);
     }
   }
   s->shape.agent_blocks = static_cast<uint32_t>(s->agent_blocks.size());
@@ -272,7 +289,7 @@ int build_launch_tables(epi_sim* s) {
     const uint32_t O = static_cast<uint32_t>(cnt.size());
     while (j < O) {
       if (cnt[j] > Bo) {
-        for (uint32_t k = 0; k < cnt[j]; k += Bo) wb.push_back(AgentBlock{i, slot + k, std::min(Bo, cnt[j] - k), j, j, 1, 0, 0});
+        for (uint32_t k = 0; k < cnt[j]; k += Bo) wb.push_back(office_block(D.agent_off, i, slot + k, std::min(Bo, cnt[j] - k), j, j, 0));
         slot += cnt[j];
         ++j;
         continue;
@@ -280,11 +297,11 @@ int build_launch_tables(epi_sim* s) {
       const uint32_t first = slot, j_lo = j;
       uint32_t count = 0;
       while (j < O && j - j_lo < kMaxFilterOffices && count + cnt[j] <= Bo) count += cnt[j++];
-      if (count) wb.push_back(AgentBlock{i, first, count, j_lo, j - 1, j_lo, j - 1, 0});
+      if (count) wb.push_back(office_block(D.agent_off, i, first, count, j_lo, j - 1, 1));
       slot += count;
     }
     for (uint32_t first = slot; first < D.n; first += Bo)
-      rb.push_back(AgentBlock{i, first, std::min(Bo, D.n - first), 1, 0, 1, 0, 0});
+      rb.push_back(office_block(D.agent_off, i, first, std::min(Bo, D.n - first), 1, 0, 0));
     const size_t total = wb.size() + rb.size();
     std::vector<AgentBlock> merged;
     merged.reserve(total);
@@ -399,18 +416,20 @@ int enqueue_hour(epi_sim* s, uint32_t next_hour) {
   return EPI_OK;
 }
 
-// Hours first..last of one day (24d+1 .. 24d+24). Hours of day 1..6 are one launch when
-// the handle allows the night launch and the range holds all six, and 3..6 one
-// epilogue-only launch when it allows quiet hours and the range holds all four.
-int enqueue_hours(epi_sim* s, uint32_t first, uint32_t last) {
+// The groups of hours that the day from `hour` + 1 on runs as one launch each.
+uint8_t flags_of_day(const epi_sim* s, uint32_t hour) { return s->day_flags[hour / 24u]; }
+
+// Hours first..last of one day (24d+1 .. 24d+24), the groups that `flags` allows and the
+// range holds whole in one launch each.
+int enqueue_hours(epi_sim* s, uint32_t first, uint32_t last, uint8_t flags) {
   for (uint32_t h = first; h <= last;) {
     const uint32_t hd = h % 24u;
-    if (s->night && hd == 1 && last - h >= 5u) {
+    if ((flags & DAY_NIGHT) && hd == 1 && last - h >= 5u) {
       HIP_TRY(launch_night(s->v, s->shape, s->stream));
       h += 6;
       continue;
     }
-    if (s->quiet_hours && hd == 3 && last - h >= 3u) {
+    if ((flags & DAY_QUIET) && hd == 3 && last - h >= 3u) {
       HIP_TRY(launch_quiet_hours(s->v, s->shape, 4, s->stream));
       h += 4;
       continue;
@@ -431,21 +450,21 @@ int enqueue_hours_plain(epi_sim* s, uint32_t first, uint32_t last) {
   return EPI_OK;
 }
 
-int capture_day_graph(epi_sim* s) {
-  if (s->day_graph) return EPI_OK;
+int capture_day_graph(epi_sim* s, uint8_t flags) {
+  if (s->day_graph[flags]) return EPI_OK;
   hipGraph_t graph = nullptr;
   HIP_TRY(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-  const int rc = enqueue_hours(s, 1, 24);  // the hours of day of 24d+1 .. 24d+24
+  const int rc = enqueue_hours(s, 1, 24, flags);  // the hours of day of 24d+1 .. 24d+24
   hipError_t e = hipStreamEndCapture(s->stream, &graph);
   if (rc != EPI_OK) {
     if (graph) (void)hipGraphDestroy(graph);
     return rc;
   }
   if (e != hipSuccess) return fail(EPI_ERR_DEVICE, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-  e = hipGraphInstantiate(&s->day_graph, graph, nullptr, nullptr, 0);
+  e = hipGraphInstantiate(&s->day_graph[flags], graph, nullptr, nullptr, 0);
   (void)hipGraphDestroy(graph);
   if (e != hipSuccess) {
-    s->day_graph = nullptr;
+    s->day_graph[flags] = nullptr;
     return fail(EPI_ERR_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
   }
   return EPI_OK;
@@ -554,13 +573,15 @@ int advance(epi_sim* s, uint32_t target) {
       if (all_inactive(s, s->pinned_active + slot * s->n_sims)) break;
     }
     if (graph_ok && s->host_hour % 24u == 0 && target - s->host_hour >= 24u) {
-      int rc = capture_day_graph(s);
+      const uint8_t flags = flags_of_day(s, s->host_hour);
+      int rc = capture_day_graph(s, flags);
       if (rc != EPI_OK) return rc;
-      HIP_TRY(hipGraphLaunch(s->day_graph, s->stream));
+      HIP_TRY(hipGraphLaunch(s->day_graph[flags], s->stream));
       s->host_hour += 24;
     } else {
       const uint32_t end = std::min(target, (s->host_hour / 24u + 1u) * 24u);
-      const int rc = graph_ok ? enqueue_hours(s, s->host_hour + 1, end) : enqueue_hours_plain(s, s->host_hour + 1, end);
+      const int rc = graph_ok ? enqueue_hours(s, s->host_hour + 1, end, flags_of_day(s, s->host_hour))
+                              : enqueue_hours_plain(s, s->host_hour + 1, end);
       if (rc != EPI_OK) return rc;
       s->host_hour = end;
     }
@@ -620,6 +641,22 @@ int step_impl(epi_sim* s, uint32_t n_hours, epi_counts* rows, uint32_t row_strid
     if (stopped) stopped[i] = st.active ? 0 : 1;
   }
   return EPI_OK;
+}
+
+void set_day_flags(epi_sim* s) {
+  s->day_flags.assign(s->max_hour / 24u + 1u, DAY_NIGHT | DAY_QUIET);
+  const auto clear = [&](uint32_t hour, uint32_t from, uint32_t to, uint8_t flag) {
+    const uint32_t hd = hour % 24u;
+    if (hour > 0 && hour <= s->max_hour && hd >= from && hd <= to) s->day_flags[(hour - 1u) / 24u] &= static_cast<uint8_t>(~flag);
+  };
+  for (uint32_t h : s->vacc_hour) {
+    clear(h, 1, 5, DAY_NIGHT);
+    clear(h, 2, 5, DAY_QUIET);
+  }
+  for (uint32_t i = 0; i < s->n_sims; ++i) {
+    const uint32_t last = s->desc[i].hours > 0 ? s->desc[i].hours - 1u : 0u;
+    clear(last, 1, 6, DAY_NIGHT);
+  }
 }
 
 int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_t>& seeds, uint32_t flags,
@@ -760,16 +797,7 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
   // overrides both, epi_set_office_block_size then the office layout's alone.
   s->shape.block = (s->n_sims == 1 && s->desc[0].n >= (1u << 19)) ? 512u : 256u;
   s->shape.office_block = s->shape.block;
-  s->quiet_hours = true;
-  s->night = true;
-  for (uint32_t h : s->vacc_hour) {
-    if (h % 24u >= 2u && h % 24u <= 5u) s->quiet_hours = false;
-    if (h % 24u >= 1u && h % 24u <= 5u) s->night = false;
-  }
-  for (uint32_t i = 0; i < s->n_sims; ++i) {
-    const uint32_t last = s->desc[i].hours > 0 ? s->desc[i].hours - 1u : 0u;
-    if (last % 24u >= 1u && last % 24u <= 6u) s->night = false;
-  }
+  set_day_flags(s.get());
 
   // device memory
   HIP_TRY(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
@@ -802,7 +830,7 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
   s->cap_office_blocks = max_office_blocks;
   HIP_TRY(M.alloc(&s->d_office_agent, s->n_agents));
   HIP_TRY(M.alloc(&s->d_office_slot, s->n_agents));
-  HIP_TRY(M.alloc(&v.block_counts, 6 * std::max(max_blocks, max_office_blocks)));
+  HIP_TRY(M.alloc(&v.block_counts, 8 * std::max(max_blocks, max_office_blocks)));
   v.agent_blocks = s->d_agent_blocks;
   BlockRef* d_hosp_blocks = nullptr;
   HIP_TRY(M.alloc(&d_hosp_blocks, s->hosp_blocks.size()));
@@ -1356,10 +1384,11 @@ static int set_launch_blocks(epi_sim* sim, uint32_t home, uint32_t office) {
   if (rc != EPI_OK) return rc;
   rc = upload_tables(sim);
   if (rc != EPI_OK) return rc;
-  if (sim->day_graph) {
-    (void)hipGraphExecDestroy(sim->day_graph);
-    sim->day_graph = nullptr;
-  }
+  for (hipGraphExec_t& g : sim->day_graph)
+    if (g) {
+      (void)hipGraphExecDestroy(g);
+      g = nullptr;
+    }
   return EPI_OK;
 }
 

@@ -16,12 +16,12 @@ namespace epi {
 
 struct FastDiv {
   uint32_t d;      // divisor, >= 1
-  uint32_t m;      // magic multiplier (unused for d == 1)
+  uint32_t m;      // magic multiplier (1 for d == 1)
   uint32_t shift;  // l - 1
 };
 
 inline FastDiv make_fastdiv(uint32_t d) {
-  FastDiv f{d, 0u, 0u};
+  FastDiv f{d, 1u, 0u};
   if (d <= 1) {
     f.d = 1;
     return f;
@@ -42,9 +42,8 @@ EPI_FD_HD uint32_t fd_mulhi(uint32_t a, uint32_t b) {
 }
 
 EPI_FD_HD uint32_t fast_div(uint32_t n, const FastDiv& f) {
-  if (f.d == 1) return n;
-  const uint32_t t = fd_mulhi(n, f.m);
-  return (t + ((n - t) >> 1)) >> f.shift;
+  const uint32_t t = fd_mulhi(n, f.m);  // 0 for d == 1, whose quotient n - t is not halved
+  return (t + ((n - t) >> (f.d != 1u ? 1u : 0u))) >> f.shift;
 }
 
 EPI_FD_HD uint32_t fast_mod(uint32_t n, const FastDiv& f) { return n - fast_div(n, f) * f.d; }

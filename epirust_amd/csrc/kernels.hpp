@@ -29,7 +29,7 @@ struct DevView {
   Event* events;
   const uint32_t* vacc_hour;
   const unsigned long long* vacc_thr;
-  uint32_t* block_counts;  // 6 per agent block: the hour's partial S E I H R D
+  uint32_t* block_counts;  // 8 per agent block: the hour's partial S E I H R D
   // Host-visible (pinned) copies that every hour's epilogue writes: its row (indexed like
   // rows) and the simulation's state after it. A step call reads them after one drain.
   Counts7* host_rows;

@@ -91,8 +91,9 @@ struct DiseaseParams {
   uint32_t hosp_window;
 };
 
-// Read-only per-simulation descriptor (device copy built once at create).
-struct SimDesc {
+// Read-only per-simulation descriptor (device copy built once at create), on cache lines of
+// its own.
+struct alignas(64) SimDesc {
   uint32_t n;          // agents
   uint32_t g;          // grid_size
   uint32_t stride;     // logical grid width (>= g+1)
@@ -130,7 +131,7 @@ struct SimDesc {
 };
 
 // Mutable per-simulation scalars, owned by the device.
-struct SimState {
+struct alignas(64) SimState {
   uint32_t hour;            // last hour stepped
   uint32_t active;          // 0 once stopped (E=I=H=0) or out of hours
   uint32_t commit_hour[2];  // [hour & 1]: the hour the agent pass of that parity runs, 0 = none
@@ -152,7 +153,6 @@ struct SimState {
   // launch (hours of day 1..6 together) applies it while its epilogues refill the slots.
   uint32_t night_sweep, night_vacc_hour;
   uint64_t night_vacc_thr;
-  uint32_t pad[2];
 };
 
 // Launch-table entry: (simulation, first hospital cell).
@@ -164,14 +164,20 @@ struct BlockRef {
 // 10 x 10 office) fits its LDS array.
 constexpr uint32_t kMaxFilterOffices = 20;
 
-// Agent-block table entry: slots first .. first + count - 1 of simulation sim. In the
-// office layout a block holds either workers of offices j_lo .. j_hi (every worker of
-// offices full_lo .. full_hi among them) or only agents that are not office workers
-// (j_lo > j_hi); in the home layout j_lo > j_hi too.
+// Agent-block table entry: slots first .. first + count - 1 of simulation sim, whose agent
+// arrays start at agent_off. In the office layout a block holds either workers of offices
+// j_lo .. j_hi (whole: every worker of them) or only agents that are not office workers (j_lo >
+// j_hi); in the home layout the same words are the simulation's fd_houses, so that a block's
+// first loads wait for its entry only.
 struct AgentBlock {
+  uint64_t agent_off;
   uint32_t sim, first, count;
-  uint32_t j_lo, j_hi, full_lo, full_hi;
-  uint32_t pad;
+  union {
+    struct {
+      uint32_t j_lo, j_hi, whole;
+    };
+    FastDiv houses;
+  };
 };
 
 struct Counts7 {
