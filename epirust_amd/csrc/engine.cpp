@@ -411,7 +411,7 @@ int enqueue_hour(epi_sim* s, uint32_t next_hour) {
     if (rc != EPI_OK) return rc;
   }
   const DevView& v = office_hour(next_hour) ? s->v_office : s->v;
-  if (hour_has_step(next_hour)) HIP_TRY(launch_step(v, s->shape, s->stream));
+  if (hour_has_step(next_hour)) HIP_TRY(launch_step(v, s->shape, next_hour, s->stream));
   HIP_TRY(launch_commit(v, s->shape, next_hour, s->stream));
   return EPI_OK;
 }
@@ -1329,7 +1329,7 @@ int epi_profile(epi_sim* sim, uint32_t n_hours, double ms_mean[3], uint32_t laun
       // the layout moves of hours of day 8 and 16 are timed with the step
       if ((h % 24u == 8 || h % 24u == 16) && rc == EPI_OK) rc = relayout(sim, h % 24u == 8);
       const DevView& v = office_hour(h) ? sim->v_office : sim->v;
-      if (had_step[k] && launch_step(v, sim->shape, sim->stream) != hipSuccess) rc = fail(EPI_ERR_DEVICE, "launch");
+      if (had_step[k] && launch_step(v, sim->shape, h, sim->stream) != hipSuccess) rc = fail(EPI_ERR_DEVICE, "launch");
       (void)hipEventRecord(e[2], sim->stream);
       if (launch_commit(v, sim->shape, h, sim->stream) != hipSuccess) rc = fail(EPI_ERR_DEVICE, "launch");
       (void)hipEventRecord(e[3], sim->stream);

@@ -66,6 +66,36 @@ constexpr uint32_t kTgtCell = ~(kTgtWon | kTgtHouse);
 constexpr uint32_t kTgtNone = ~0u;
 constexpr uint32_t kMaxWaves = 16;  // of a block of 1,024 threads
 
+// k_step is compiled once per class of hours of day that take the same branches of the
+// routine: every test of the hour folds, and with it the code of the other hours (static
+// VALU / SALU instructions and scalar loads of an evening hour: 1,314 / 1,180 / 79 in one
+// kernel for all hours, 832 / 556 / 37 in its own), which shortens what a small simulation's
+// few waves wait for (10k agents 7.64 -> 7.25 us an hour, 100k 8.57 -> 8.31).
+enum HourClass : uint32_t {
+  HOURS_0,      // hospital admission
+  HOURS_7_17,   // public transport, the others stay
+  HOURS_8,      // to work
+  HOURS_9_15,   // in the office; non-workers in the housing area until 12, at home after
+  HOURS_16,     // home
+  HOURS_18_22,  // where one is
+  HOURS_23      // recovery or death
+};
+constexpr uint32_t first_hour(HourClass c) {
+  return c == HOURS_0 ? 0u : c == HOURS_7_17 ? 7u : c == HOURS_8 ? 8u : c == HOURS_9_15 ? 9u : c == HOURS_16 ? 16u
+         : c == HOURS_18_22 ? 18u : 23u;
+}
+constexpr uint32_t last_hour(HourClass c) {
+  return c == HOURS_7_17 ? 17u : c == HOURS_9_15 ? 15u : c == HOURS_18_22 ? 22u : first_hour(c);
+}
+constexpr bool on_office_layout(HourClass c) { return c == HOURS_8 || c == HOURS_9_15; }
+// Whether an hour of day of class C is `at`.
+template <HourClass C>
+__device__ __forceinline__ bool is_hour(uint32_t hd, uint32_t at) {
+  if (at < first_hour(C) || at > last_hour(C)) return false;
+  if (C == HOURS_7_17 && at != 7u && at != 17u) return false;
+  return first_hour(C) == last_hour(C) || hd == at;
+}
+
 // Hour of day 2: block b of a simulation's n_blocks resets its share of the claim array
 // (all padded cells, in 16-byte stores; the array of each simulation is a multiple of 4
 // cells long and starts at a multiple of 4). The share is computed before the block's
@@ -333,13 +363,14 @@ struct Agent {
 
   // citizen/mod.rs:257-349: choose the primitive and the area it leads to, run it, then the
   // disease update (skipped by the hospital-staff quarantine transitions, which return early).
+  template <HourClass C>
   __device__ __forceinline__ void perform_movements(uint32_t hd) {
     const uint32_t s = ws();
     uint32_t act = ACT_NONE, new_area = ~0u;
     Rect target = D.housing;
     bool disease = true;
     if (s == WS_NORMAL || s == WS_ESSENTIAL) {
-      if (hd == 7 || hd == 17) {
+      if (C == HOURS_7_17) {
         if (w & F_PT) {
           target = D.transport;
           act = tele_act(target);
@@ -347,11 +378,11 @@ struct Agent {
         } else {
           act = ACT_LOCAL;
         }
-      } else if (hd == 8) {
+      } else if (is_hour<C>(hd, 8)) {
         target = work();
         act = tele_act(target);
         new_area = AREA_WORK;
-      } else if (hd == 16) {
+      } else if (is_hour<C>(hd, 16)) {
         target = home();
         act = tele_act(target);
         new_area = AREA_HOME;
@@ -369,7 +400,7 @@ struct Agent {
         new_area = AREA_HOME;
         wsa = h + 24u * 14u;
         disease = false;
-      } else if (hd == 8) {
+      } else if (is_hour<C>(hd, 8)) {
         const uint32_t ver = S.hosp_version;
         if (!same_rect(current_area(), D.hosp[ver]) && wsa <= h) {
           target = D.hosp[ver];
@@ -378,15 +409,15 @@ struct Agent {
           wsa = h;
         }
         w &= ~F_WQ;
-      } else if (hd == 16) {
+      } else if (is_hour<C>(hd, 16)) {
         w |= F_WQ;
       } else if (!(w & F_WQ)) {
         act = ACT_LOCAL;
       }
     } else {  // NA: goto_area of a non-worker is move_agent_from in the current area
       act = ACT_LOCAL;
-      if (hd == 8) new_area = AREA_HOUSING;
-      else if (hd == 12) new_area = AREA_HOME;
+      if (is_hour<C>(hd, 8)) new_area = AREA_HOUSING;
+      else if (is_hour<C>(hd, 12)) new_area = AREA_HOME;
     }
     move(act, target);
     if (new_area != ~0u) set_area(new_area);
@@ -623,7 +654,12 @@ __device__ __forceinline__ void epilogue_block(const DevView& v, uint32_t sim) {
   }
 }
 
-__global__ void k_step(DevView v) {
+// 80 scalar registers: a wave takes 16 more than its code, in steps of 16 out of 800 a SIMD, so
+// the 90 that most classes would take leave six waves of a 512-thread block's two per SIMD where
+// eight fit (10M agents 166 -> 158 us an hour, 1M 20.2 -> 19.6).
+template <HourClass C>
+__global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(DevView v) {
+  constexpr bool office = on_office_layout(C);
   const AgentBlock bm = scalar_copy(v.agent_blocks + blockIdx.x);
   const uint32_t count = first_lane(bm.count);
   // Every slot below the block's count holds an agent (the office slot map is a
@@ -634,7 +670,7 @@ __global__ void k_step(DevView v) {
   const uint32_t slot = first_lane(bm.first) + min(threadIdx.x, count - 1u);
   const uint64_t gi = bm.agent_off + slot;
   uint32_t local = slot, w_stored = v.st[gi], p = v.pos[gi];  // the agent id, its words
-  if (v.office) local = v.office_agent[gi];  // uniform
+  if (office) local = v.office_agent[gi];  // uniform
   const uint32_t sim = first_lane(bm.sim);
   const SimDesc& D = v.desc[sim];
   SimState* S = v.state + sim;
@@ -654,7 +690,7 @@ __global__ void k_step(DevView v) {
   // Office hours: the offices of this block's workers (j_lo .. j_hi, none in a block of
   // other agents and in the home layout), each with 100 cells in the block's claim filter.
   const uint32_t j_lo = first_lane(bm.j_lo), j_hi = first_lane(bm.j_hi);
-  const bool filter = v.office && j_lo <= j_hi && (j_hi - j_lo + 1u) <= kMaxFilterOffices;
+  const bool filter = office && j_lo <= j_hi && (j_hi - j_lo + 1u) <= kMaxFilterOffices;
   if (valid) {
     // st and pos are loaded together, then the work that needs neither (the buildings and
     // the hour's movement draw, which hours of day 0 and 23 do not use: hospitalize draws it
@@ -663,8 +699,8 @@ __global__ void k_step(DevView v) {
     Agent a(D, *S, occ);
     a.id = local;
     a.h = h;
-    a.locate_buildings(hd >= 8 && hd <= 16);
-    if (hd != 0 && hd != 23) a.mv = a.dr(SITE_MOVE, 0);
+    a.locate_buildings(office || C == HOURS_16);
+    if (C != HOURS_0 && C != HOURS_23) a.mv = a.dr(SITE_MOVE, 0);
     loaded_together(w_stored, p, a.mv);
     a.w = sweep.mask ? apply_sweep(w_stored, sweep, local, D) : w_stored;
     a.x = static_cast<int32_t>(p & 0xFFFFu);
@@ -679,17 +715,17 @@ __global__ void k_step(DevView v) {
     a.wsa = staff ? v.wsa[gid] : 0u;
     const uint32_t wsa0 = a.wsa;
 
-    if (Disease::draws_needed(a.w, hd)) a.dz = a.dr(SITE_DISEASE, 0);
-    if (hd == 0) {
+    if (Disease::draws_needed(a.w, first_hour(C) == last_hour(C) ? first_hour(C) : hd)) a.dz = a.dr(SITE_DISEASE, 0);
+    if constexpr (C == HOURS_0) {
       if (a.state() == ST_I) {  // increment_infection_day (state.rs:69-73)
         const uint32_t day = fld(a.w, B_DAY, M_DAY);
         a.w = set_fld(a.w, B_DAY, M_DAY, day < kMaxDay ? day + 1 : day);
       }
       a.hospitalize();
-    } else if (hd == 23) {
+    } else if constexpr (C == HOURS_23) {
       a.deceased();
     } else {
-      a.perform_movements(hd);
+      a.perform_movements<C>(hd);
     }
     // Everything the stores need is computed first: a descriptor field read after a store
     // can no longer come from the scalar cache and costs a vector round trip.
@@ -721,7 +757,7 @@ __global__ void k_step(DevView v) {
     // hospital fallback at 0) are its own agents'; no one has the housing area then. So
     // the lowest-id claimant of such a cell is found among the agent's lower housemates,
     // whose target words the commit reads: no global claim is made.
-    house_move = !v.office && moves && a.in_house(a.tx, a.ty);
+    house_move = !office && moves && a.in_house(a.tx, a.ty);
     if (a.tm != a.tm0) v.tm[gid] = a.tm;
     if (staff && a.wsa != wsa0) v.wsa[gid] = a.wsa;
   }
@@ -802,7 +838,7 @@ __global__ void k_quiet_hours(DevView v, uint32_t n_hours) {
 // epilogues rewrite the parity slots meanwhile, so the agent blocks read hour of day 0's
 // sweep from its own slot, and whether the simulation runs from `active`, which these
 // hours cannot change (counts repeat, and a day graph never holds the last hour).
-__global__ void k_night(DevView v, uint32_t n_epi) {
+__global__ __attribute__((amdgpu_num_sgpr(80))) void k_night(DevView v, uint32_t n_epi) {
   if (blockIdx.x < n_epi) {  // uniform
     if (threadIdx.x == 0) quiet_epilogues(v, blockIdx.x, 6);
     return;
@@ -1082,11 +1118,26 @@ hipError_t launch_hospital_scan(const DevView& v, const LaunchShape& s, hipStrea
   return hipGetLastError();
 }
 
-hipError_t launch_step(const DevView& v, const LaunchShape& s, hipStream_t stream) {
-  const uint32_t blocks = v.office ? s.office_agent_blocks : s.agent_blocks;
-  if (blocks == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_step, dim3(blocks), dim3(v.office ? s.office_block : s.block), 0, stream, v);
+template <HourClass C>
+hipError_t launch_step_class(const DevView& v, uint32_t blocks, uint32_t threads, hipStream_t stream) {
+  hipLaunchKernelGGL(k_step<C>, dim3(blocks), dim3(threads), 0, stream, v);
   return hipGetLastError();
+}
+
+hipError_t launch_step(const DevView& v, const LaunchShape& s, uint32_t hour, hipStream_t stream) {
+  const uint32_t blocks = v.office ? s.office_agent_blocks : s.agent_blocks;
+  const uint32_t threads = v.office ? s.office_block : s.block;
+  if (blocks == 0) return hipSuccess;
+  switch (hour % 24u) {
+    case 0: return launch_step_class<HOURS_0>(v, blocks, threads, stream);
+    case 7: case 17: return launch_step_class<HOURS_7_17>(v, blocks, threads, stream);
+    case 8: return launch_step_class<HOURS_8>(v, blocks, threads, stream);
+    case 16: return launch_step_class<HOURS_16>(v, blocks, threads, stream);
+    case 23: return launch_step_class<HOURS_23>(v, blocks, threads, stream);
+    default:
+      return v.office ? launch_step_class<HOURS_9_15>(v, blocks, threads, stream)
+                      : launch_step_class<HOURS_18_22>(v, blocks, threads, stream);
+  }
 }
 
 hipError_t launch_commit(const DevView& v, const LaunchShape& s, uint32_t hour, hipStream_t stream) {
