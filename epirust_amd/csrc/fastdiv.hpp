@@ -43,7 +43,7 @@ EPI_FD_HD uint32_t fd_mulhi(uint32_t a, uint32_t b) {
 
 EPI_FD_HD uint32_t fast_div(uint32_t n, const FastDiv& f) {
   const uint32_t t = fd_mulhi(n, f.m);  // 0 for d == 1, whose quotient n - t is not halved
-  return (t + ((n - t) >> (f.d != 1u ? 1u : 0u))) >> f.shift;
+  return (t + ((n - t) >> (f.d - 1u < 1u ? f.d - 1u : 1u))) >> f.shift;
 }
 
 EPI_FD_HD uint32_t fast_mod(uint32_t n, const FastDiv& f) { return n - fast_div(n, f) * f.d; }

@@ -64,6 +64,7 @@ constexpr uint32_t kTgtHouse = 1u << 15;
 constexpr uint32_t kTgtCell = ~(kTgtWon | kTgtHouse);
 // A non-mover: its cell part (x = y = 32767) is no cell, so it equals no move's word.
 constexpr uint32_t kTgtNone = ~0u;
+constexpr uint32_t kNoState = 5u;  // in the state bits of a lane without an agent
 constexpr uint32_t kMaxWaves = 16;  // of a block of 1,024 threads
 
 // k_step is compiled once per class of hours of day that take the same branches of the
@@ -129,12 +130,12 @@ struct Agent {
   int32_t hx = 0, hy = 0;           // home house origin (house id % H)
   int32_t ox = 0, oy = 0;           // office origin (office id % O)
   // The hour's movement and disease draw blocks, computed once up front (one inlined
-  // Philox each) for the hours / states that can use them.
-  u32x4 mv{{0, 0, 0, 0}}, dz{{0, 0, 0, 0}};
-  // 5x5 grid window around (wx, wy), one 64-bit row per grid row: bytes of columns
-  // c0 .. c0+7 where c0 = (x + kPadX - 2) & ~3 and woff = x + kPadX - c0 (2..5).
-  bool have_win = false;
-  int32_t wx = 0, wy = 0, woff = 0;
+  // Philox each) for the hours / states that can use them; the movement's last round is left
+  // to the words that are read (all but a few agents read one).
+  Philox9 mv{};
+  u32x4 dz{{0, 0, 0, 0}};
+  // 5x5 grid window around (wx, wy): the eight bytes of each row from column wx - 2 on.
+  int32_t wx = 0, wy = 0;
   uint64_t r0 = 0, r1 = 0, r2 = 0, r3 = 0, r4 = 0;  // named, so no variable-index access exists
 
   __device__ Agent(const SimDesc& d, const SimState& s, const uint8_t* o)
@@ -144,17 +145,18 @@ struct Agent {
   __device__ __forceinline__ u32x4 dr(uint32_t site, uint32_t block) const {
     return philox4x32_10(id, h, site, block, D.seed_lo, D.seed_hi);
   }
-  __device__ __forceinline__ const u32x4& move_words() const { return mv; }
+  __device__ __forceinline__ void draw_move() { mv = philox4x32_9(id, h, SITE_MOVE, D.seed_lo, D.seed_hi); }
   __device__ __forceinline__ const u32x4& disease_words() const { return dz; }
 
   __device__ __forceinline__ uint32_t state() const { return fld(w, B_STATE, M_STATE); }
   __device__ __forceinline__ uint32_t sev() const { return fld(w, B_SEV, M_SEV); }
   __device__ __forceinline__ uint32_t ws() const { return fld(w, B_WS, M_WS); }
   __device__ __forceinline__ bool symptomatic() const {
-    return state() == ST_I && (sev() == SEV_MILD || sev() == SEV_SEVERE);
+    static_assert(SEV_MILD == 2 && SEV_SEVERE == 3, "both have the field's high bit set");
+    return (w & ((M_STATE << B_STATE) | (2u << B_SEV))) == ((ST_I << B_STATE) | (2u << B_SEV));
   }
   __device__ __forceinline__ bool can_move() const {  // citizen/mod.rs:452-454
-    return !(symptomatic() || (w & F_HOSP) || state() == ST_D || (w & F_ISO));
+    return !(symptomatic() || (w & (F_HOSP | F_ISO)) || state() == ST_D);
   }
   // Home house id % H and office id % O, tiled row-major (area.rs:95-117), once per hour
   // with the division constants of the tiling. The office is needed only at hours of day
@@ -174,20 +176,21 @@ struct Agent {
   }
   __device__ __forceinline__ Rect home() const { return Rect{hx, hy, hx + 1, hy + 1}; }
   __device__ __forceinline__ bool in_house(int32_t cx, int32_t cy) const {
-    return cx >= hx && cx <= hx + 1 && cy >= hy && cy <= hy + 1;
+    return static_cast<uint32_t>((cx - hx) | (cy - hy)) <= 1u;
   }
   __device__ __forceinline__ Rect work() const {  // non-workers' work location is home
     return ws() == WS_NA ? home() : Rect{ox, oy, ox + 9, oy + 9};
   }
   __device__ __forceinline__ Rect area_rect(uint32_t tag) const {
-    switch (tag) {
-      case AREA_HOME: return home();
-      case AREA_WORK: return work();
-      case AREA_TRANSPORT: return D.transport;
-      case AREA_HOUSING: return D.housing;
-      case AREA_HOSP0: return D.hosp[0];
-      default: return D.hosp[1];
+    Rect a = home();
+    if (tag != AREA_HOME) {
+      if (tag == AREA_WORK) a = work();
+      else if (tag == AREA_TRANSPORT) a = D.transport;
+      else if (tag == AREA_HOUSING) a = D.housing;
+      else if (tag == AREA_HOSP0) a = D.hosp[0];
+      else a = D.hosp[1];
     }
+    return a;
   }
   __device__ __forceinline__ Rect current_area() const { return area_rect(fld(w, B_AREA, M_AREA)); }
   __device__ __forceinline__ void set_area(uint32_t tag) { w = set_fld(w, B_AREA, M_AREA, tag); }
@@ -195,61 +198,42 @@ struct Agent {
   __device__ __forceinline__ bool vacant(int32_t cx, int32_t cy) const {
     return occ[cell_index(D, cx, cy)] == 0;
   }
-  // 3 x 3 mask of the cells around (cx, cy) that lie in rect a and in the grid
-  // (area.rs:83-88 and allocation_map.rs:156-159 for each neighbour).
-  __device__ __forceinline__ uint32_t allowed9(const Rect& a, int32_t cx, int32_t cy) const {
+  // The cells around (cx, cy) that lie in rect a and in the grid (area.rs:83-88 and
+  // allocation_map.rs:156-159 for each neighbour), in the order of the eight neighbours.
+  // Areas start at coordinates >= 0 but may end past the grid.
+  __device__ __forceinline__ uint32_t allowed8(const Rect& a, int32_t cx, int32_t cy) const {
     const int32_t last = static_cast<int32_t>(D.g) - 1;
-    const uint32_t cols = span3(cx - 1, max(a.x0, 0), min(a.x1, last));
-    const uint32_t rows = span3(cy - 1, max(a.y0, 0), min(a.y1, last));
-    return cols * ((rows & 1u) | ((rows & 2u) << 2) | ((rows & 4u) << 4));  // cols copied to each row
+    const int32_t x1 = min(a.x1, last), y1 = min(a.y1, last);
+    if ((cx >= a.x0) & (cx <= x1) & (cy >= a.y0) & (cy <= y1))  // nearly always: only the edges' neighbours are out
+      return 0xFFu & ~((cx == a.x0 ? kMooreLeft : 0u) | (cx == x1 ? kMooreRight : 0u) |
+                       (cy == a.y0 ? kMooreTop : 0u) | (cy == y1 ? kMooreBottom : 0u));
+    const uint32_t cols = span3(cx - 1, a.x0, x1), rows = span3(cy - 1, a.y0, y1);
+    return moore8(cols * ((rows & 1u) | ((rows & 2u) << 2) | ((rows & 4u) << 4)));  // cols copied to each row
   }
-  __device__ __forceinline__ bool in_grid(int32_t cx, int32_t cy) const {
-    return cx >= 0 && cy >= 0 && cx < static_cast<int32_t>(D.g) && cy < static_cast<int32_t>(D.g);
-  }
-  // Ten independent aligned dword loads: rows cy-2..cy+2, 8 bytes each.
+  // Five independent loads of the two aligned words that hold columns cx-2..cx+2 of a row (an
+  // unaligned eight-byte load takes twice the L1 accesses: 10M agents 161 us an hour, 153 with
+  // these), from one offset on five uniform row bases, then shifted to column cx-2.
   __device__ __forceinline__ void load_window(int32_t cx, int32_t cy) {
-    const uint32_t px = static_cast<uint32_t>(cx) + kPadX;
-    const uint32_t c0 = (px - 2u) & ~3u;
-    const uint32_t* p = reinterpret_cast<const uint32_t*>(occ + ((static_cast<uint32_t>(cy) + kPadY - 2u) * D.pitch + c0));
-    const uint32_t q = D.pitch >> 2;
-    uint32_t lo[5], hi[5];
+    const uint32_t px = static_cast<uint32_t>(cx) + (kPadX - 2u);
+    const uint32_t off = __umul24(static_cast<uint32_t>(cy) + (kPadY - 2u), D.pitch) + (px & ~3u);
+    uint2 q[5];
 #pragma unroll
-    for (int r = 0; r < 5; ++r) {
-      lo[r] = p[r * q];
-      hi[r] = p[r * q + 1];
-    }
-    r0 = join64(hi[0], lo[0]);
-    r1 = join64(hi[1], lo[1]);
-    r2 = join64(hi[2], lo[2]);
-    r3 = join64(hi[3], lo[3]);
-    r4 = join64(hi[4], lo[4]);
+    for (uint32_t r = 0; r < 5; ++r) q[r] = load_words2(uniform_base(occ + r * D.pitch), off);
+    r0 = from_byte(q[0], px & 3u);
+    r1 = from_byte(q[1], px & 3u);
+    r2 = from_byte(q[2], px & 3u);
+    r3 = from_byte(q[3], px & 3u);
+    r4 = from_byte(q[4], px & 3u);
     wx = cx;
     wy = cy;
-    woff = static_cast<int32_t>(px - c0);
-    have_win = true;
-  }
-  template <int R>
-  __device__ __forceinline__ uint64_t row() const {
-    static_assert(R >= 0 && R < 5, "window row");
-    if constexpr (R == 0) return r0;
-    else if constexpr (R == 1) return r1;
-    else if constexpr (R == 2) return r2;
-    else if constexpr (R == 3) return r3;
-    else return r4;
-  }
-  // Byte of cell (wx + dx, wy + DY), |dx| <= 2, |DY| <= 2.
-  template <int DY>
-  __device__ __forceinline__ uint32_t wbyte(int32_t dx) const {
-    return static_cast<uint32_t>(row<DY + 2>() >> (8 * (woff + dx))) & 0xFFu;
   }
   // Make the window cover the 3x3 neighbourhood of (cx, cy).
   __device__ __forceinline__ void cover(int32_t cx, int32_t cy) {
-    if (!have_win || cx - wx > 1 || wx - cx > 1 || cy - wy > 1 || wy - cy > 1) load_window(cx, cy);
+    if (static_cast<uint32_t>(cx - wx + 1) > 2u || static_cast<uint32_t>(cy - wy + 1) > 2u) load_window(cx, cy);
   }
   __device__ __forceinline__ void random_point(const Rect& a, int32_t& px, int32_t& py) {  // area.rs:76-81
-    const u32x4& m = move_words();
-    px = a.x0 + static_cast<int32_t>(below(m.w[0], static_cast<uint32_t>(a.x1 - a.x0 + 1)));
-    py = a.y0 + static_cast<int32_t>(below(m.w[1], static_cast<uint32_t>(a.y1 - a.y0 + 1)));
+    px = a.x0 + static_cast<int32_t>(below(mv.word0(), static_cast<uint32_t>(a.x1 - a.x0 + 1)));
+    py = a.y0 + static_cast<int32_t>(below(mv.word1(), static_cast<uint32_t>(a.y1 - a.y0 + 1)));
   }
   // move_agent (allocation_map.rs:136-142): the target if vacant in the snapshot, else stay
   __device__ __forceinline__ void move_to(int32_t px, int32_t py) {
@@ -274,28 +258,30 @@ struct Agent {
     return (can_move() || override_movement) ? ACT_TELE : ACT_NONE;
   }
 
-  __device__ __forceinline__ void move(uint32_t act, const Rect& target) {
-    if (act == ACT_NONE) return;
-    const bool tele = act == ACT_TELE;
-    if (!tele && !can_move()) return;
-    const Rect a = tele ? target : current_area();
+  // Every lane takes the window of the cell that it may move from, or of its own when it stays
+  // (the infection scan reads it), so that the common case has no branches. A wave of an
+  // evening hour issues 345 vector instructions, 415 with a path per case (10M agents 158 -> 151
+  // us an hour, 1M 19.6 -> 18.9, 32 runs of 100k 48.9 -> 45.4; loads through L1 bound it next).
+  // `tag` is the area of the move: the target's for ACT_TELE, else the current one.
+  __device__ __forceinline__ void move(uint32_t act, uint32_t tag) {
+    const bool tele = act == ACT_TELE, local = (act == ACT_LOCAL) & can_move();
+    const Rect a = area_rect(tag);
     int32_t lx = x, ly = y;
-    if (tele || !contains(a, x, y)) random_point(a, lx, ly);  // teleport origin, vacancy not checked
+    if (tele | (local & !contains(a, x, y))) random_point(a, lx, ly);  // vacancy not checked
     load_window(lx, ly);
-    if (tele) {  // vacancy of the point; the window also serves the infection scan around it
-      if (wbyte<0>(0) == 0) { tx = lx; ty = ly; }
-      return;
-    }
-    // vacant Moore neighbours of (lx, ly) in the area and the grid: the window rows
-    // ly-1 .. ly+1, bytes woff-1 .. woff+1, tested as three bytes at a time
-    const uint32_t vac9 = zero3(three(r1, woff - 1)) | (zero3(three(r2, woff - 1)) << 3) |
-                          (zero3(three(r3, woff - 1)) << 6);
-    uint32_t cand = moore8(vac9 & allowed9(a, lx, ly));
+    // vacant Moore neighbours of (lx, ly) in the area and the grid: bytes 1..3 of the rows
+    // ly-1 .. ly+1
+    const uint32_t cand = local ? vacant8(r1, r2, r3) & allowed8(a, lx, ly) : 0u;
     const uint32_t n = __builtin_popcount(cand);
-    if (n == 0) return;
-    const int k = static_cast<int>(nth_bit8(cand, below(move_words().w[2], n)));
-    tx = lx + moore_dx(k);
-    ty = ly + moore_dy(k);
+    const uint32_t k = nth_bit8(cand, below(mv.word2(), n));
+    if (n != 0) {
+      tx = lx + moore_dx(k);
+      ty = ly + moore_dy(k);
+    }
+    if (tele & ((static_cast<uint32_t>(r2) & 0xFF0000u) == 0)) {  // the point itself
+      tx = lx;
+      ty = ly;
+    }
   }
 
   // default_disease_handler.rs:64-86 as an OR over fixed per-neighbour draws: first the
@@ -309,7 +295,7 @@ struct Agent {
     // No infectious cell (byte >= 2) anywhere in the 5 x 5 window, a superset of the
     // neighbourhood: nothing to test, and no draw is made. Most agents, and whole waves,
     // take this exit while infections are rare.
-    if (((r0 | r1 | r2 | r3 | r4) & 0xFEFEFEFEFEFEFEFEull) == 0) return false;
+    if (((r0 | r1 | r2 | r3 | r4) & 0xFEFEFEFEFEull) == 0) return false;
     const int32_t ox = tx - wx, oy = ty - wy;  // both in [-1, 1]
     const uint64_t mm = oy < 0 ? ~0ull : 0ull, m0 = oy == 0 ? ~0ull : 0ull, mp = oy > 0 ? ~0ull : 0ull;
     const uint64_t top = (r0 & mm) | (r1 & m0) | (r2 & mp);
@@ -317,13 +303,11 @@ struct Agent {
     const uint64_t bot = (r2 & mm) | (r3 & m0) | (r4 & mp);
     // infectious neighbours (grid byte >= 2, i.e. a byte with a bit above bit 0) and the
     // high-window ones (byte 3) among the cells of the area and the grid
-    const int32_t c = woff + ox - 1;
+    const uint32_t c = static_cast<uint32_t>(ox + 1);
     const uint32_t bt = three(top, c), bm = three(mid, c), bb = three(bot, c);
-    const uint32_t ok = allowed9(a, tx, ty);
-    uint32_t hot = moore8((nonzero3(bt & 0xFEFEFEu) | (nonzero3(bm & 0xFEFEFEu) << 3) |
-                           (nonzero3(bb & 0xFEFEFEu) << 6)) & ok);
-    const uint32_t high = moore8((nonzero3(bt & (bt >> 1) & 0x010101u) | (nonzero3(bm & (bm >> 1) & 0x010101u) << 3) |
-                                  (nonzero3(bb & (bb >> 1) & 0x010101u) << 6)) & ok);
+    const uint32_t ok = allowed8(a, tx, ty);
+    uint32_t hot = pack8(bt >> 1, bm >> 1, bb >> 1) & ok;
+    const uint32_t high = pack8(bt & (bt >> 1), bm & (bm >> 1), bb & (bb >> 1)) & ok;
     int blk = -1;
     uint32_t q0 = 0, q1 = 0, q2 = 0, q3 = 0;
     while (hot) {
@@ -365,47 +349,25 @@ struct Agent {
   // disease update (skipped by the hospital-staff quarantine transitions, which return early).
   template <HourClass C>
   __device__ __forceinline__ void perform_movements(uint32_t hd) {
-    const uint32_t s = ws();
-    uint32_t act = ACT_NONE, new_area = ~0u;
-    Rect target = D.housing;
+    const uint32_t s = ws(), here = fld(w, B_AREA, M_AREA);
+    uint32_t act = ACT_LOCAL, tag = here;
     bool disease = true;
-    if (s == WS_NORMAL || s == WS_ESSENTIAL) {
-      if (C == HOURS_7_17) {
-        if (w & F_PT) {
-          target = D.transport;
-          act = tele_act(target);
-          new_area = AREA_TRANSPORT;
-        } else {
-          act = ACT_LOCAL;
-        }
-      } else if (is_hour<C>(hd, 8)) {
-        target = work();
-        act = tele_act(target);
-        new_area = AREA_WORK;
-      } else if (is_hour<C>(hd, 16)) {
-        target = home();
-        act = tele_act(target);
-        new_area = AREA_HOME;
-      } else {
-        act = ACT_LOCAL;
-      }
-    } else if (s == WS_STAFF) {
+    if (s == WS_STAFF) {
       const uint32_t since = h > wsa ? h - wsa : 0u;  // saturating_sub
+      act = ACT_NONE;
       if (since == 24u * 14u) {
         w |= F_WQ;
         disease = false;
       } else if (since == 24u * 14u * 2u) {
-        target = home();
-        act = tele_act(target);
-        new_area = AREA_HOME;
+        act = tele_act(home());
+        tag = AREA_HOME;
         wsa = h + 24u * 14u;
         disease = false;
       } else if (is_hour<C>(hd, 8)) {
         const uint32_t ver = S.hosp_version;
         if (!same_rect(current_area(), D.hosp[ver]) && wsa <= h) {
-          target = D.hosp[ver];
-          act = tele_act(target);
-          new_area = AREA_HOSP0 + ver;
+          act = tele_act(D.hosp[ver]);
+          tag = AREA_HOSP0 + ver;
           wsa = h;
         }
         w &= ~F_WQ;
@@ -414,13 +376,23 @@ struct Agent {
       } else if (!(w & F_WQ)) {
         act = ACT_LOCAL;
       }
-    } else {  // NA: goto_area of a non-worker is move_agent_from in the current area
-      act = ACT_LOCAL;
-      if (is_hour<C>(hd, 8)) new_area = AREA_HOUSING;
-      else if (is_hour<C>(hd, 12)) new_area = AREA_HOME;
+    } else if (s != WS_NA) {
+      if (C == HOURS_7_17 && (w & F_PT)) {
+        act = tele_act(D.transport);
+        tag = AREA_TRANSPORT;
+      } else if (is_hour<C>(hd, 8)) {
+        act = can_move() ? ACT_TELE : ACT_NONE;  // an office is no home
+        tag = AREA_WORK;
+      } else if (is_hour<C>(hd, 16)) {
+        act = tele_act(home());
+        tag = AREA_HOME;
+      }
     }
-    move(act, target);
-    if (new_area != ~0u) set_area(new_area);
+    move(act, tag);
+    // goto_area of a non-worker is move_agent_from in the area it is still in
+    if (s == WS_NA && is_hour<C>(hd, 8)) tag = AREA_HOUSING;
+    if (s == WS_NA && is_hour<C>(hd, 12)) tag = AREA_HOME;
+    if (tag != here) set_area(tag);
     if (disease) update_infection_dynamics();
   }
 
@@ -435,7 +407,7 @@ struct Agent {
       ty = hr.y0 + static_cast<int32_t>(fv / wd);
       w |= F_HOSP;
     } else {
-      mv = dr(SITE_MOVE, 0);  // hour of day 0 draws it only here
+      draw_move();  // hour of day 0 draws it only here
       int32_t px, py;
       random_point(home(), px, py);
       move_to(px, py);
@@ -448,7 +420,7 @@ struct Agent {
     load_tm();
     Disease::on_routine_end(D.dz, disease_words(), w, tm);
     if (state() == ST_R) {
-      mv = dr(SITE_MOVE, 0);  // hour of day 23 draws it only here
+      draw_move();  // hour of day 23 draws it only here
       int32_t px, py;
       random_point(home(), px, py);
       move_to(px, py);
@@ -667,23 +639,25 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(DevView v) {
   // agent words are loaded alongside it, and alongside the descriptor; lanes past the count
   // read the block's last agent.
   const bool valid = threadIdx.x < count;
-  const uint32_t slot = first_lane(bm.first) + min(threadIdx.x, count - 1u);
-  const uint64_t gi = bm.agent_off + slot;
-  uint32_t local = slot, w_stored = v.st[gi], p = v.pos[gi];  // the agent id, its words
-  if (office) local = v.office_agent[gi];  // uniform
+  const uint32_t lane_slot = min(threadIdx.x, count - 1u);
+  const uint64_t g0 = bm.agent_off + first_lane(bm.first);
+  uint32_t local = first_lane(bm.first) + lane_slot;  // the agent id, its words
+  uint32_t w_stored = (v.st + g0)[lane_slot], p = (v.pos + g0)[lane_slot];
+  if (office) local = (v.office_agent + g0)[lane_slot];
   const uint32_t sim = first_lane(bm.sim);
   const SimDesc& D = v.desc[sim];
   SimState* S = v.state + sim;
   if (!S->active) return;  // uniform over the block
   const uint32_t h = S->hour + 1;  // an hour of day 0 or 7..23
-  const uint32_t hd = h % 24u;
+  const uint32_t hd = first_hour(C) == last_hour(C) ? first_hour(C) : h % 24u;
+  constexpr uint32_t kFirst = first_hour(C), kLast = last_hour(C);
+  __builtin_assume(hd >= kFirst && hd <= kLast);
   const Sweep sweep = sweep_slot(*S, (h - 1u) & 1u);  // decided at hour h - 1
   const uint8_t* occ = v.occ + D.cell_off;
 
-  uint32_t cat = 6;
   // This lane's claim and state word, carried past the block's claim filter to the stores.
   bool moves = false;
-  uint32_t key = 0, w_out = 0, w_in = 0, tgt_word = 0, office_cell = kNoCell;
+  uint32_t key = 0, w_out = kNoState, w_in = kNoState, tgt_word = 0, office_cell = kNoCell;
   bool whole_office = false;  // the claimed cell's office has all its slots in this block
   bool house_move = false;    // a home-layout move into the agent's own house
   uint64_t ci = 0;
@@ -700,7 +674,7 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(DevView v) {
     a.id = local;
     a.h = h;
     a.locate_buildings(office || C == HOURS_16);
-    if (C != HOURS_0 && C != HOURS_23) a.mv = a.dr(SITE_MOVE, 0);
+    if (C != HOURS_0 && C != HOURS_23) a.draw_move();
     loaded_together(w_stored, p, a.mv);
     a.w = sweep.mask ? apply_sweep(w_stored, sweep, local, D) : w_stored;
     a.x = static_cast<int32_t>(p & 0xFFFFu);
@@ -715,7 +689,7 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(DevView v) {
     a.wsa = staff ? v.wsa[gid] : 0u;
     const uint32_t wsa0 = a.wsa;
 
-    if (Disease::draws_needed(a.w, first_hour(C) == last_hour(C) ? first_hour(C) : hd)) a.dz = a.dr(SITE_DISEASE, 0);
+    if (Disease::draws_needed(a.w, hd)) a.dz = a.dr(SITE_DISEASE, 0);
     if constexpr (C == HOURS_0) {
       if (a.state() == ST_I) {  // increment_infection_day (state.rs:69-73)
         const uint32_t day = fld(a.w, B_DAY, M_DAY);
@@ -730,17 +704,15 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(DevView v) {
     // Everything the stores need is computed first: a descriptor field read after a store
     // can no longer come from the scalar cache and costs a vector round trip.
     key = claim_key(h, local);
-    moves = a.tx != a.x || a.ty != a.y;
+    tgt_word = static_cast<uint32_t>(a.tx) | (static_cast<uint32_t>(a.ty) << 16);
+    moves = tgt_word != p;
     // the grid byte depends only on the state, the hospitalized flag, the infection day and
     // the immunity, so it is recomputed only when one of those changed this hour
     constexpr uint32_t kByteFields = (M_STATE << B_STATE) | F_HOSP | (M_DAY << B_DAY) | (M_IMM << B_IMM);
     if (((a.w ^ w0) & kByteFields) && occupant_byte(D.dz, a.w) != occupant_byte(D.dz, w0)) a.w |= F_DIRTY;
     ci = D.cell_off + cell_index(D, a.tx, a.ty);
-    const uint32_t s = a.state();
-    cat = s == ST_S ? 0u : s == ST_E ? 1u : s == ST_I ? ((a.w & F_HOSP) ? 3u : 2u) : s == ST_R ? 4u : 5u;
     w_out = a.w;
     w_in = w0;
-    tgt_word = static_cast<uint32_t>(a.tx) | (static_cast<uint32_t>(a.ty) << 16);
     // a worker's claim of a cell of its own office (the only agents that claim office
     // cells at these hours) enters the filter
     const uint32_t j = fast_mod(local, D.fd_offices);  // the agent's office
@@ -783,20 +755,24 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(DevView v) {
       else if (house_move) tgt_word |= kTgtHouse;
       else atomicMin(&v.claim[ci], key);
     }
-    v.tgt[gi] = moves ? tgt_word : kTgtNone;
-    if (w_out != w_in) v.st[gi] = w_out;
+    (v.tgt + g0)[lane_slot] = moves ? tgt_word : kTgtNone;
+    if (w_out != w_in) (v.st + g0)[lane_slot] = w_out;
   }
 
-  // S/E/I/H/R/D via wavefront ballots, each wave's into its own LDS words (nothing to clear
-  // first), then one plain store per block and category; the epilogue adds up the blocks'.
+  // S/E/I/H/R/D from the wave's masks of the state's bits, each wave's into its own LDS words
+  // (nothing to clear first), then one plain store per block and category; the epilogue adds up
+  // the blocks'. Lanes without an agent hold no state.
+  static_assert(ST_S == 0 && ST_E == 1 && ST_I == 2 && ST_R == 3 && ST_D == 4 && kNoState == 5 && B_STATE == 0, "bits");
   __shared__ uint32_t s_counts[kMaxWaves][8];
   const uint32_t lane = threadIdx.x & (kWave - 1);
-  uint32_t mine = 0;
-#pragma unroll
-  for (uint32_t k = 0; k < 6; ++k) {
-    const uint32_t n = static_cast<uint32_t>(__popcll(__ballot(cat == k)));
-    mine = lane == k ? n : mine;
-  }
+  const uint64_t b0 = __ballot(w_out & 1u), b1 = __ballot(w_out & 2u), b2 = __ballot(w_out & 4u);
+  const uint64_t in_hospital = __ballot(w_out & F_HOSP), infected = b1 & ~b0;
+  uint32_t mine = wave_count(~(b0 | b1 | b2));
+  mine = lane_word<1>(mine, wave_count(b0 & ~(b1 | b2)));
+  mine = lane_word<2>(mine, wave_count(infected & ~in_hospital));
+  mine = lane_word<3>(mine, wave_count(infected & in_hospital));
+  mine = lane_word<4>(mine, wave_count(b0 & b1));
+  mine = lane_word<5>(mine, wave_count(b2 & ~b0));
   if (lane < 6) s_counts[threadIdx.x / kWave][lane] = mine;
   __syncthreads();
   if (threadIdx.x < 6) {

@@ -55,6 +55,57 @@ EPI_HD u32x4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, u
   return u32x4{{c0, c1, c2, c3}};
 }
 
+// Nine of the ten rounds of the block (c0, c1, c2, 0), and its words 0..2, each by the part
+// of the last round that it needs. c1 and c2 are uniform on the device: what the first two
+// rounds make of them is plain arithmetic that the scalar unit can do.
+struct Philox9 {
+  uint32_t c0, c1, c2, c3, k0, k1;  // before the last round
+  EPI_HD uint32_t word0() const {
+    uint32_t hi, lo;
+    mulhilo32(0xCD9E8D57u, c2, hi, lo);
+    return xor3(hi, c1, k0);
+  }
+  EPI_HD uint32_t word1() const { return 0xCD9E8D57u * c2; }
+  EPI_HD uint32_t word2() const {
+    uint32_t hi, lo;
+    mulhilo32(0xD2511F53u, c0, hi, lo);
+    return xor3(hi, c3, k1);
+  }
+};
+EPI_HD Philox9 philox4x32_9(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t k0, uint32_t k1) {
+  uint32_t hi0, lo0, hi1, lo1;
+  mulhilo32(0xD2511F53u, c0, hi0, lo0);
+  mulhilo32(0xCD9E8D57u, c2, hi1, lo1);  // constant
+  const uint32_t u = hi1 ^ c1 ^ k0;      // uniform
+  c2 = hi0 ^ k1;
+  c1 = lo1;
+  uint32_t c3 = lo0;
+  k0 += 0x9E3779B9u;
+  k1 += 0xBB67AE85u;
+  mulhilo32(0xD2511F53u, u, hi0, lo0);  // uniform
+  mulhilo32(0xCD9E8D57u, c2, hi1, lo1);
+  c0 = hi1 ^ (c1 ^ k0);
+  c2 = c3 ^ (hi0 ^ k1);
+  c1 = lo1;
+  c3 = lo0;
+  k0 += 0x9E3779B9u;
+  k1 += 0xBB67AE85u;
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+#endif
+  for (int r = 2; r < 9; ++r) {
+    mulhilo32(0xD2511F53u, c0, hi0, lo0);
+    mulhilo32(0xCD9E8D57u, c2, hi1, lo1);
+    c0 = xor3(hi1, c1, k0);
+    c2 = r == 2 ? hi0 ^ (c3 ^ k1) : xor3(hi0, c3, k1);
+    c1 = lo1;
+    c3 = lo0;
+    k0 += 0x9E3779B9u;
+    k1 += 0xBB67AE85u;
+  }
+  return Philox9{c0, c1, c2, c3, k0, k1};
+}
+
 // One draw block for (seed, id, hour, site, block).
 EPI_HD u32x4 draw(uint64_t seed, uint32_t id, uint32_t hour, uint32_t site, uint32_t block) {
   return philox4x32_10(id, hour, site, block, static_cast<uint32_t>(seed), static_cast<uint32_t>(seed >> 32));

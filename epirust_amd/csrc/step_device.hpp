@@ -41,8 +41,8 @@ __device__ __forceinline__ void loaded_together(uint32_t& a, uint32_t& b, uint32
 }
 // The same for two loaded words and a draw block computed while they are in flight: the
 // draw's words pass through the barrier too, so its rounds are scheduled before the wait.
-__device__ __forceinline__ void loaded_together(uint32_t& a, uint32_t& b, u32x4& d) {
-  asm("" : "+v"(a), "+v"(b), "+v"(d.w[0]), "+v"(d.w[1]), "+v"(d.w[2]), "+v"(d.w[3]));
+__device__ __forceinline__ void loaded_together(uint32_t& a, uint32_t& b, Philox9& d) {
+  asm("" : "+v"(a), "+v"(b), "+v"(d.c0), "+v"(d.c1), "+v"(d.c2), "+v"(d.c3));
 }
 
 // Sum over the wave, in lane 63: adds across lanes by DPP (rows of 16, then their last lanes
@@ -61,29 +61,30 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
   return x;
 }
 
+// Lanes set in a wave's mask, and `x` with lane `lane` replaced, both on the scalar unit.
+__device__ __forceinline__ uint32_t wave_count(uint64_t mask) { return static_cast<uint32_t>(__builtin_popcountll(mask)); }
+template <int LANE>
+__device__ __forceinline__ uint32_t lane_word(uint32_t x, uint32_t value) {
+  asm("v_writelane_b32 %0, %1, %2" : "+v"(x) : "s"(value), "n"(LANE));
+  return x;
+}
+
 __device__ __forceinline__ bool contains(const Rect& a, int32_t x, int32_t y) {
-  return a.x0 <= x && a.x1 >= x && a.y0 <= y && a.y1 >= y;
+  return (a.x0 <= x) & (a.x1 >= x) & (a.y0 <= y) & (a.y1 >= y);  // no branches
 }
 __device__ __forceinline__ bool same_rect(const Rect& a, const Rect& b) {
   return a.x0 == b.x0 && a.y0 == b.y0 && a.x1 == b.x1 && a.y1 == b.y1;
 }
 
-// Moore neighbour order (point.rs:57-61): (-1,-1) (0,-1) (1,-1) (-1,0) (1,0) (-1,1) (0,1) (1,1)
-__device__ constexpr int moore_dx(int k) { return k < 3 ? k - 1 : (k == 3 ? -1 : (k == 4 ? 1 : k - 6)); }
-__device__ constexpr int moore_dy(int k) { return k < 3 ? -1 : (k < 5 ? 0 : 1); }
-
-// Compile-time loop over the eight Moore neighbours: f(Idx<k>) for k = 0..7.
-template <int V>
-struct Idx {
-  static constexpr int value = V;
-};
-template <int K = 0, class F>
-__device__ __forceinline__ void for_moore(F&& f) {
-  if constexpr (K < 8) {
-    f(Idx<K>{});
-    for_moore<K + 1>(f);
-  }
+// Moore neighbour order (point.rs:57-61): (-1,-1) (0,-1) (1,-1) (-1,0) (1,0) (-1,1) (0,1) (1,1),
+// offsets as two-bit fields of a constant, and the neighbours of each edge as eight bits.
+__device__ __forceinline__ int32_t moore_dx(uint32_t k) {
+  return static_cast<int32_t>((0x9224u >> (2u * k)) & 3u) - 1;
 }
+__device__ __forceinline__ int32_t moore_dy(uint32_t k) {
+  return static_cast<int32_t>((0xA940u >> (2u * k)) & 3u) - 1;
+}
+constexpr uint32_t kMooreLeft = 0x29u, kMooreRight = 0x94u, kMooreTop = 0x07u, kMooreBottom = 0xE0u;
 
 __device__ __forceinline__ uint32_t fld(uint32_t w, uint32_t b, uint32_t m) { return (w >> b) & m; }
 __device__ __forceinline__ uint32_t set_fld(uint32_t w, uint32_t b, uint32_t m, uint32_t v) {
@@ -94,7 +95,7 @@ __device__ __forceinline__ uint32_t set_fld(uint32_t w, uint32_t b, uint32_t m, 
 // has fewer than 2^32 padded cells (grid_size <= 32,000), so the index is 32-bit and a
 // load adds it to the simulation's base as an unsigned offset.
 __device__ __forceinline__ uint32_t cell_index(uint32_t pitch, int32_t x, int32_t y) {
-  return (static_cast<uint32_t>(y) + kPadY) * pitch + static_cast<uint32_t>(x) + kPadX;
+  return __umul24(static_cast<uint32_t>(y) + kPadY, pitch) + static_cast<uint32_t>(x) + kPadX;
 }
 __device__ __forceinline__ uint32_t cell_index(const SimDesc& D, int32_t x, int32_t y) {
   return cell_index(D.pitch, x, y);
@@ -131,19 +132,45 @@ __device__ __forceinline__ uint32_t span3(int32_t base, int32_t lo, int32_t hi) 
   return (0x7u << from) & (0x7u >> past) & 0x7u;
 }
 
-// Three grid bytes as 24 bits (columns px-1, px, px+1 of a window row).
-__device__ __forceinline__ uint32_t three(uint64_t row, int32_t byte_off) {
-  return static_cast<uint32_t>(row >> (8 * byte_off)) & 0xFFFFFFu;
+// A pointer that is the same in all lanes, kept in scalar registers: a load adds the lane's
+// 32-bit offset to it in the instruction, where the compiler would otherwise fold the pointer
+// into the lane's part and pay a 64-bit vector add per load.
+typedef const __attribute__((address_space(1))) uint8_t* GlobalBytes;
+__device__ __forceinline__ GlobalBytes uniform_base(const uint8_t* p) {
+  GlobalBytes q = (GlobalBytes)p;
+  asm("" : "+s"(q));
+  return q;
 }
-// Per-byte tests of three bytes, each to bits 0..2. Exact: adding 0x7F to a byte's low
-// seven bits never carries into the next byte.
-__device__ __forceinline__ uint32_t pack3(uint32_t top_bits) {  // bits 7, 15, 23 -> 0, 1, 2
-  return ((top_bits >> 7) & 1u) | ((top_bits >> 14) & 2u) | ((top_bits >> 21) & 4u);
+// Two words at base + off, off a multiple of 4.
+__device__ __forceinline__ uint2 load_words2(GlobalBytes base, uint32_t off) {
+  typedef uint64_t Words __attribute__((aligned(4)));
+  const uint64_t q = *reinterpret_cast<const __attribute__((address_space(1))) Words*>(base + off);
+  return make_uint2(static_cast<uint32_t>(q), static_cast<uint32_t>(q >> 32));
 }
-__device__ __forceinline__ uint32_t nonzero3(uint32_t v) {
-  return pack3((((v & 0x7F7F7Fu) + 0x7F7F7Fu) | v) & 0x808080u);
+// The bytes of q from byte `first` (0..3) on.
+__device__ __forceinline__ uint64_t from_byte(uint2 q, uint32_t first) {
+  return join64(q.y >> (8u * first), __builtin_amdgcn_alignbyte(q.y, q.x, first));
 }
-__device__ __forceinline__ uint32_t zero3(uint32_t v) { return nonzero3(v) ^ 0x7u; }
+// Bytes `first` .. first + 3 (first <= 3) of a window row: columns px-1, px, px+1 and one more.
+__device__ __forceinline__ uint32_t three(uint64_t row, uint32_t first) {
+  return __builtin_amdgcn_alignbyte(static_cast<uint32_t>(row >> 32), static_cast<uint32_t>(row), first);
+}
+// Bit 0 of the low three bytes of three words (rows y-1, y, y+1) as the eight neighbours, the
+// centre dropped: products with byte weights, added up.
+__device__ __forceinline__ uint32_t pack8(uint32_t top, uint32_t mid, uint32_t bottom) {
+  constexpr uint32_t kBit0 = 0x01010101u;
+  return __builtin_amdgcn_udot4(
+      top & kBit0, 0x00040201u,
+      __builtin_amdgcn_udot4(mid & kBit0, 0x00100008u,
+                             __builtin_amdgcn_udot4(bottom & kBit0, 0x00804020u, 0u, false), false),
+      false);
+}
+// The vacant ones among the eight neighbours of the cell in byte 2 of the middle row; a
+// grid byte is 0..3, so a cell is occupied iff one of its two low bits is set.
+__device__ __forceinline__ uint32_t vacant8(uint64_t above, uint64_t row, uint64_t below) {
+  const uint32_t t = three(above, 1), m = three(row, 1), b = three(below, 1);
+  return pack8(t | (t >> 1), m | (m >> 1), b | (b >> 1)) ^ 0xFFu;
+}
 
 // Claim key of agent `id` at `hour`: hours of day 7..23, 0 (the hours that move anyone)
 // rank 0..17 since the reset at hour of day 2; a later hour takes a smaller top field, so
