@@ -32,7 +32,9 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 COMMON = ["-std=c++17", "-O3", "-fPIC", "-Wall", "-I" + SRC, "-I" + os.path.join(ROOT, "include")]
 HOST = ["-I" + os.path.join(ROCM, "include"), "-D__HIP_PLATFORM_AMD__"]
 # Packed FP32 instructions are kept out of every code object built here.
-DEVICE = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# The first 16 words of a kernel's scalar arguments arrive in registers with the wave.
+DEVICE = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+          "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
 HOST_SOURCES = ["config.cpp", "population.cpp", "engine.cpp", "cli.cpp", "mlp_engine.cpp"]
 DEVICE_SOURCES = ["kernels.hip", "init.hip", "stream.hip", "mlp.hip"]

@@ -455,12 +455,13 @@ struct EpilogueIn {
   unsigned long long vacc_t;
 };
 
-__device__ __forceinline__ void load_epilogue_in(const DevView& v, uint32_t sim, EpilogueIn& in) {
-  const SimDesc d = scalar_copy(v.desc + sim);
+__device__ __forceinline__ void load_epilogue_in(const DevView& v, const SimDesc* desc, const SimState* state,
+                                                 uint32_t sim, EpilogueIn& in) {
+  const SimDesc d = scalar_copy(desc + sim);
   in.D = EpiDesc{d.row_off, d.event_off, d.event_cap, d.hours, d.n_vacc, d.vacc_off,
                  d.has_lockdown, d.lockdown_at, d.has_hospital, d.spread_rate_threshold,
                  v.office ? d.office_block_begin : d.block_begin, v.office ? d.office_n_blocks : d.n_blocks};
-  in.st = scalar_copy(v.state + sim);
+  in.st = scalar_copy(state + sim);
   const bool more = in.st.vacc_next < in.D.n_vacc;
   in.vacc_h = more ? scalar_copy(v.vacc_hour + in.D.vacc_off + in.st.vacc_next) : ~0u;
   in.vacc_t = more ? scalar_copy(v.vacc_thr + in.D.vacc_off + in.st.vacc_next) : 0ull;
@@ -588,14 +589,16 @@ __device__ __forceinline__ void add_partials(uint32_t (&acc)[6], const uint32_t*
 // DPP and one barrier; the state is worked on in registers and written once. With the step's
 // and commit's agent words loaded right after the table entry, an hour of 10k agents took
 // 8.60 -> 7.72 us, of 100k 9.69 -> 8.68 and of 1M 21.2 -> 20.4.
-__device__ __forceinline__ void epilogue_block(const DevView& v, uint32_t sim) {
+template <bool ONE>
+__device__ __forceinline__ void epilogue_block(const DevView& v, const SimDesc* desc, SimState* state, uint32_t block) {
+  const uint32_t sim = ONE ? 0u : block;
   __shared__ uint32_t s_sum[kMaxWaves][8];
   EpilogueIn in;
-  load_epilogue_in(v, sim, in);  // uniform: scalar registers
+  load_epilogue_in(v, desc, state, sim, in);  // uniform: scalar registers
   if (!in.st.active) {           // uniform
     if (threadIdx.x == 0) {
       clear_commit_slot(in.st);
-      v.state[sim] = in.st;
+      state[sim] = in.st;
     }
     return;
   }
@@ -606,7 +609,7 @@ __device__ __forceinline__ void epilogue_block(const DevView& v, uint32_t sim) {
     for (int k = 0; k < 6; ++k) c[k] = in.st.last_counts[k];
   } else {
     uint32_t acc[6] = {0, 0, 0, 0, 0, 0};
-    add_partials(acc, v.block_counts + 8ull * in.D.block_begin, in.D.n_blocks);
+    add_partials(acc, v.block_counts + 8ull * (ONE ? 0u : in.D.block_begin), in.D.n_blocks);
     // Each wave's six sums to its own LDS words, then thread 0 adds up the waves'.
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
@@ -629,10 +632,16 @@ __device__ __forceinline__ void epilogue_block(const DevView& v, uint32_t sim) {
 // 80 scalar registers: a wave takes 16 more than its code, in steps of 16 out of 800 a SIMD, so
 // the 90 that most classes would take leave six waves of a 512-thread block's two per SIMD where
 // eight fit (10M agents 166 -> 158 us an hour, 1M 20.2 -> 19.6).
-template <HourClass C>
-__global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(DevView v) {
+// The first arguments repeat fields of the view: they arrive in registers with the wave
+// (kernel argument preload). ONE: the view has one simulation, whose descriptor and state need
+// not wait for the block's entry to name it. With both, an hour of 10k agents takes 7.08 -> 6.99
+// us, of 100k 7.99 -> 7.90, of 10M 150.9 -> 149.7 (with the preload alone 7.06, 8.00, 150.3).
+template <HourClass C, bool ONE>
+__global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(const AgentBlock* blocks, const SimDesc* desc,
+                                                            SimState* state, const uint32_t* st, const uint32_t* pos,
+                                                            const uint32_t* ids, DevView v) {
   constexpr bool office = on_office_layout(C);
-  const AgentBlock bm = scalar_copy(v.agent_blocks + blockIdx.x);
+  const AgentBlock bm = scalar_copy(blocks + blockIdx.x);
   const uint32_t count = first_lane(bm.count);
   // Every slot below the block's count holds an agent (the office slot map is a
   // permutation of the ids), so validity does not wait for the slot -> id read, and the
@@ -640,14 +649,14 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(DevView v) {
   // read the block's last agent.
   const bool valid = threadIdx.x < count;
   const uint32_t lane_slot = min(threadIdx.x, count - 1u);
-  const uint64_t g0 = bm.agent_off + first_lane(bm.first);
+  const uint64_t g0 = (ONE ? 0ull : bm.agent_off) + first_lane(bm.first);
   uint32_t local = first_lane(bm.first) + lane_slot;  // the agent id, its words
-  uint32_t w_stored = (v.st + g0)[lane_slot], p = (v.pos + g0)[lane_slot];
-  if (office) local = (v.office_agent + g0)[lane_slot];
-  const uint32_t sim = first_lane(bm.sim);
-  const SimDesc& D = v.desc[sim];
-  SimState* S = v.state + sim;
-  if (!S->active) return;  // uniform over the block
+  uint32_t w_stored = (st + g0)[lane_slot], p = (pos + g0)[lane_slot];
+  if (office) local = (ids + g0)[lane_slot];
+  const uint32_t sim = ONE ? 0u : first_lane(bm.sim);
+  const SimDesc& D = desc[sim];
+  SimState* S = state + sim;
+  uint32_t active = S->active;
   const uint32_t h = S->hour + 1;  // an hour of day 0 or 7..23
   const uint32_t hd = first_hour(C) == last_hour(C) ? first_hour(C) : h % 24u;
   constexpr uint32_t kFirst = first_hour(C), kLast = last_hour(C);
@@ -665,17 +674,18 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(DevView v) {
   // other agents and in the home layout), each with 100 cells in the block's claim filter.
   const uint32_t j_lo = first_lane(bm.j_lo), j_hi = first_lane(bm.j_hi);
   const bool filter = office && j_lo <= j_hi && (j_hi - j_lo + 1u) <= kMaxFilterOffices;
+  // st and pos are in flight while the work that needs neither is done (the buildings and the
+  // hour's movement draw, which hours of day 0 and 23 do not use: hospitalize draws it for its
+  // rare fallback, deceased for the recovered, who go home), then one wait (wsa and tm are read
+  // by few agents and loaded where they are needed).
+  Agent a(D, *S, occ);
+  a.id = local;
+  a.h = h;
+  a.locate_buildings(office || C == HOURS_16);
+  if (C != HOURS_0 && C != HOURS_23) a.draw_move();
+  loaded_together(w_stored, p, a.mv, active);
+  if (!active) return;  // uniform over the block
   if (valid) {
-    // st and pos are loaded together, then the work that needs neither (the buildings and
-    // the hour's movement draw, which hours of day 0 and 23 do not use: hospitalize draws it
-    // for its rare fallback, deceased for the recovered, who go home), then one wait (wsa
-    // and tm are read by few agents and loaded where they are needed).
-    Agent a(D, *S, occ);
-    a.id = local;
-    a.h = h;
-    a.locate_buildings(office || C == HOURS_16);
-    if (C != HOURS_0 && C != HOURS_23) a.draw_move();
-    loaded_together(w_stored, p, a.mv);
     a.w = sweep.mask ? apply_sweep(w_stored, sweep, local, D) : w_stored;
     a.x = static_cast<int32_t>(p & 0xFFFFu);
     a.y = static_cast<int32_t>(p >> 16);
@@ -789,7 +799,7 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(DevView v) {
 // what epilogue_block does for it.
 __device__ void quiet_epilogues(const DevView& v, uint32_t sim, uint32_t n_hours) {
   EpilogueIn in;
-  load_epilogue_in(v, sim, in);
+  load_epilogue_in(v, v.desc, v.state, sim, in);
   for (uint32_t k = 0; k < n_hours; ++k) {
     if (!in.st.active) {
       clear_commit_slot(in.st);
@@ -863,22 +873,27 @@ __device__ __forceinline__ void rest_pass(const DevView& v, const SimDesc& D, co
 // the commit at hours of day 0 and 7..23, rest_pass at 1..6. Eight waves per SIMD (64 VGPRs)
 // for the agent pass, whose waves mostly wait for the grid: with the 98 VGPRs that the
 // epilogue would take, an hour of 10M agents takes 177 us instead of 160.
-__global__ __attribute__((amdgpu_waves_per_eu(8))) void k_commit(DevView v, uint32_t parity, uint32_t n_epi) {
-  if (blockIdx.x < n_epi) {  // uniform
-    epilogue_block(v, blockIdx.x);
+// Arguments and ONE as in k_step.
+template <bool ONE>
+__global__ __attribute__((amdgpu_waves_per_eu(8))) void k_commit(const AgentBlock* blocks, const SimDesc* desc,
+                                                                 SimState* state, uint32_t* st, uint32_t* pos,
+                                                                 const uint32_t* tgt, uint32_t parity, uint32_t n_epi,
+                                                                 DevView v) {
+  if (blockIdx.x < (ONE ? 1u : n_epi)) {  // uniform
+    epilogue_block<ONE>(v, desc, state, blockIdx.x);
     return;
   }
-  const AgentBlock bm = scalar_copy(v.agent_blocks + (blockIdx.x - n_epi));
+  const AgentBlock bm = scalar_copy(blocks + (blockIdx.x - (ONE ? 1u : n_epi)));
   const uint32_t count = first_lane(bm.count);
   const uint32_t slot = first_lane(bm.first) + min(threadIdx.x, count - 1u);  // as in k_step
-  const uint64_t gi = bm.agent_off + slot;
+  const uint64_t gi = (ONE ? 0ull : bm.agent_off) + slot;
   // st, pos and tgt are loaded together, and at home-layout hours with them the target
   // words of the agent's lower housemates (ids local - k * n_houses, k = 1..3: a house
   // holds at most 4 agents, grid.rs:133-142), consecutive for consecutive ids. A house
   // move then pays one round trip; a claimed move two (these words, then its claim).
-  uint32_t w = v.st[gi];
-  uint32_t p = v.pos[gi];
-  uint32_t t = v.tgt[gi];
+  uint32_t w = st[gi];
+  uint32_t p = pos[gi];
+  uint32_t t = tgt[gi];
   uint32_t local = slot;  // the agent id
   uint32_t m1 = kTgtNone, m2 = kTgtNone, m3 = kTgtNone;
   if (v.office) {  // uniform
@@ -886,22 +901,22 @@ __global__ __attribute__((amdgpu_waves_per_eu(8))) void k_commit(DevView v, uint
   } else {
     const uint32_t lower = fast_div(slot, bm.houses);  // lower housemates
     const uint32_t H = bm.houses.d;
-    if (lower >= 1) m1 = v.tgt[gi - H];
-    if (lower >= 2) m2 = v.tgt[gi - 2ull * H];
-    if (lower >= 3) m3 = v.tgt[gi - 3ull * H];
+    if (lower >= 1) m1 = tgt[gi - H];
+    if (lower >= 2) m2 = tgt[gi - 2ull * H];
+    if (lower >= 3) m3 = tgt[gi - 3ull * H];
   }
-  const uint32_t sim = first_lane(bm.sim);
-  const SimDesc& D = v.desc[sim];
-  const SimState* S = v.state + sim;
-  const uint32_t h = scalar_copy(&S->commit_hour[parity]);
+  const uint32_t sim = ONE ? 0u : first_lane(bm.sim);
+  const SimDesc& D = desc[sim];
+  const SimState* S = state + sim;
+  uint32_t h = scalar_copy(&S->commit_hour[parity]);
+  loaded_together(m1, m2, m3);
+  loaded_together(w, p, t, h);
   if (h == 0) return;  // uniform: the simulation did not step this hour
   if (h % 24u >= 1 && h % 24u <= 6) {  // uniform; home layout
-    rest_pass(v, D, *S, h, first_lane(bm.first) + threadIdx.x, blockIdx.x - n_epi - D.block_begin);
+    rest_pass(v, D, *S, h, first_lane(bm.first) + threadIdx.x, blockIdx.x - (ONE ? 1u : n_epi) - D.block_begin);
     return;
   }
   if (threadIdx.x < count) {
-    loaded_together(m1, m2, m3);
-    loaded_together(w, p, t);
     const bool mover = t != kTgtNone;
     if (mover || (w & F_DIRTY)) {
       const uint64_t cell_off = scalar_copy(&D.cell_off);
@@ -922,12 +937,12 @@ __global__ __attribute__((amdgpu_waves_per_eu(8))) void k_commit(DevView v, uint
         if (won || (!house && (v.claim + cell_off)[ci] == claim_key(h, local))) {
           occ[old_ci] = 0;
           occ[ci] = byte;
-          v.pos[gi] = t;
+          pos[gi] = t;
           moved = true;
         }
       }
       if (!moved && (w & F_DIRTY)) occ[old_ci] = byte;
-      if (w & F_DIRTY) v.st[gi] = w & ~F_DIRTY;
+      if (w & F_DIRTY) st[gi] = w & ~F_DIRTY;
     }
   }
 }
@@ -1095,8 +1110,11 @@ hipError_t launch_hospital_scan(const DevView& v, const LaunchShape& s, hipStrea
 }
 
 template <HourClass C>
-hipError_t launch_step_class(const DevView& v, uint32_t blocks, uint32_t threads, hipStream_t stream) {
-  hipLaunchKernelGGL(k_step<C>, dim3(blocks), dim3(threads), 0, stream, v);
+hipError_t launch_step_class(const DevView& v, const LaunchShape& s, uint32_t blocks, uint32_t threads,
+                             hipStream_t stream) {
+  const auto kernel = s.n_sims == 1 ? k_step<C, true> : k_step<C, false>;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, stream, v.agent_blocks, v.desc, v.state, v.st, v.pos,
+                     v.office_agent, v);
   return hipGetLastError();
 }
 
@@ -1105,22 +1123,23 @@ hipError_t launch_step(const DevView& v, const LaunchShape& s, uint32_t hour, hi
   const uint32_t threads = v.office ? s.office_block : s.block;
   if (blocks == 0) return hipSuccess;
   switch (hour % 24u) {
-    case 0: return launch_step_class<HOURS_0>(v, blocks, threads, stream);
-    case 7: case 17: return launch_step_class<HOURS_7_17>(v, blocks, threads, stream);
-    case 8: return launch_step_class<HOURS_8>(v, blocks, threads, stream);
-    case 16: return launch_step_class<HOURS_16>(v, blocks, threads, stream);
-    case 23: return launch_step_class<HOURS_23>(v, blocks, threads, stream);
+    case 0: return launch_step_class<HOURS_0>(v, s, blocks, threads, stream);
+    case 7: case 17: return launch_step_class<HOURS_7_17>(v, s, blocks, threads, stream);
+    case 8: return launch_step_class<HOURS_8>(v, s, blocks, threads, stream);
+    case 16: return launch_step_class<HOURS_16>(v, s, blocks, threads, stream);
+    case 23: return launch_step_class<HOURS_23>(v, s, blocks, threads, stream);
     default:
-      return v.office ? launch_step_class<HOURS_9_15>(v, blocks, threads, stream)
-                      : launch_step_class<HOURS_18_22>(v, blocks, threads, stream);
+      return v.office ? launch_step_class<HOURS_9_15>(v, s, blocks, threads, stream)
+                      : launch_step_class<HOURS_18_22>(v, s, blocks, threads, stream);
   }
 }
 
 hipError_t launch_commit(const DevView& v, const LaunchShape& s, uint32_t hour, hipStream_t stream) {
   const uint32_t blocks = v.office ? s.office_agent_blocks : s.agent_blocks;
   if (blocks + s.n_sims == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_commit, dim3(s.n_sims + blocks), dim3(v.office ? s.office_block : s.block), 0, stream, v,
-                     hour & 1u, s.n_sims);
+  const auto kernel = s.n_sims == 1 ? k_commit<true> : k_commit<false>;
+  hipLaunchKernelGGL(kernel, dim3(s.n_sims + blocks), dim3(v.office ? s.office_block : s.block), 0, stream,
+                     v.agent_blocks, v.desc, v.state, v.st, v.pos, v.tgt, hour & 1u, s.n_sims, v);
   return hipGetLastError();
 }
 

@@ -39,10 +39,15 @@ __device__ __forceinline__ T scalar_copy(const T* p) {
 __device__ __forceinline__ void loaded_together(uint32_t& a, uint32_t& b, uint32_t& c) {
   asm("" : "+v"(a), "+v"(b), "+v"(c));
 }
-// The same for two loaded words and a draw block computed while they are in flight: the
+// The same with a uniform word that the next branch tests: it passes through too, so the loads
+// are not sunk behind the branch (and behind the wait for that word).
+__device__ __forceinline__ void loaded_together(uint32_t& a, uint32_t& b, uint32_t& c, uint32_t& uniform) {
+  asm("" : "+v"(a), "+v"(b), "+v"(c), "+s"(uniform));
+}
+// And for two loaded words and a draw block computed while they are in flight: the
 // draw's words pass through the barrier too, so its rounds are scheduled before the wait.
-__device__ __forceinline__ void loaded_together(uint32_t& a, uint32_t& b, Philox9& d) {
-  asm("" : "+v"(a), "+v"(b), "+v"(d.c0), "+v"(d.c1), "+v"(d.c2), "+v"(d.c3));
+__device__ __forceinline__ void loaded_together(uint32_t& a, uint32_t& b, Philox9& d, uint32_t& uniform) {
+  asm("" : "+v"(a), "+v"(b), "+v"(d.c0), "+v"(d.c1), "+v"(d.c2), "+v"(d.c3), "+s"(uniform));
 }
 
 // Sum over the wave, in lane 63: adds across lanes by DPP (rows of 16, then their last lanes
