@@ -332,16 +332,21 @@ int build_launch_tables(epi_sim* s) {
 // other agents in id order. Work statuses are fixed at creation, so the slot maps are
 // built once, on the device from the synthesized state words, with the layout move's tiles.
 int build_office_order(epi_sim* s) {
-  s->office_workers.assign(s->n_sims, {});
+  std::vector<OfficeJob> jobs;
+  for (uint32_t i = 0; i < s->n_sims; ++i) {
+    const SimDesc& D = s->desc[i];
+    jobs.push_back(OfficeJob{D.n, D.n_offices, s->v.st + D.agent_off, s->d_office_agent + D.agent_off,
+                             s->d_office_slot + D.agent_off});
+  }
+  std::string err;
+  const hipError_t e = build_office_maps_on_device(jobs, s->office_workers, s->stream, err);
+  if (e != hipSuccess) return fail(EPI_ERR_DEVICE, "office layout (" + err + "): " + hipGetErrorString(e));
   std::vector<TileRef> tiles;
   for (uint32_t i = 0; i < s->n_sims; ++i) {
     SimDesc& D = s->desc[i];
     const uint32_t n = D.n, O = D.n_offices;
-    std::string err;
-    const hipError_t e = build_office_maps_on_device(s->v.st + D.agent_off, n, O, s->d_office_agent + D.agent_off,
-                                                     s->d_office_slot + D.agent_off, s->office_workers[i],
-                                                     D.n_workers, s->stream, err);
-    if (e != hipSuccess) return fail(EPI_ERR_DEVICE, "office layout (" + err + "): " + hipGetErrorString(e));
+    D.n_workers = 0;
+    for (uint32_t c : s->office_workers[i]) D.n_workers += c;
     // Tiles column by column (32 offices, every k), so that consecutive tiles share the
     // cache lines of their office slots: an office's workers, split over a column's k
     // tiles, and the other agents of neighbouring columns, whose slots follow id order.
@@ -845,6 +850,7 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
   v.vacc_thr = d_vacc_thr;
 
   std::vector<uint8_t> grid;
+  std::vector<InitJob> jobs;
   for (uint32_t i = 0; i < s->n_sims; ++i) {
     const SimDesc& D = s->desc[i];
     const Population& P = pops[i];
@@ -857,11 +863,8 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
     st.first_vacant = ~0u;
     s->state_h[i] = st;
     if (!host_init) {
-      const InitTargets t{v.pos + D.agent_off, v.st + D.agent_off, v.tm + D.agent_off, v.wsa + D.agent_off,
-                          v.occ + D.cell_off, D.pitch, padded_cells(P.geo.stride, P.geo.height)};
-      std::string err;
-      const hipError_t e = synthesize_on_device(s->cfg[i], s->seed[i], P.geo, t, s->stream, err);
-      if (e != hipSuccess) return fail(EPI_ERR_DEVICE, "device population synthesis (" + err + "): " + hipGetErrorString(e));
+      jobs.push_back(InitJob{&s->cfg[i], s->seed[i], &P.geo, v.pos + D.agent_off, v.st + D.agent_off,
+                             v.tm + D.agent_off, v.wsa + D.agent_off, v.occ + D.cell_off, D.pitch});
       continue;
     }
     if (D.n) {
@@ -878,6 +881,12 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
           occupant_byte(D.dz, P.st[a]);
     }
     HIP_TRY(hipMemcpy(v.occ + D.cell_off, grid.data(), cells, hipMemcpyHostToDevice));
+  }
+  if (!jobs.empty()) {
+    HIP_TRY(hipMemsetAsync(v.occ, 0, s->n_cells, s->stream));
+    std::string err;
+    const hipError_t e = synthesize_on_device(jobs, s->stream, err);
+    if (e != hipSuccess) return fail(EPI_ERR_DEVICE, "device population synthesis (" + err + "): " + hipGetErrorString(e));
   }
   HIP_TRY(hipMemcpy(v.state, s->state_h.data(), s->n_sims * sizeof(SimState), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_hosp_blocks, s->hosp_blocks.data(), s->hosp_blocks.size() * sizeof(BlockRef),

@@ -3,25 +3,30 @@
 // The reference builds the population on the CPU (engine/src/geography/grid.rs:83-155,
 // engine/src/citizen/citizen_factory.rs:31-134, epidemiology_simulation.rs:75-192); in
 // deterministic mode every draw is a Philox block at hour 0xFFFFFFFF, so each step is a
-// data-parallel kernel over agents or houses:
+// data-parallel kernel over agents or houses of every simulation of a batch at once (a block
+// finds its simulation in a table of first blocks, in which it searches by halving):
 //   k_init_agents  : per agent, working / public transport / work status / immunity
 //                    (sites INIT_A, INIT_B, INIT_C); the public-transport draw is kept in
 //                    F_PT and counted per block;
-//   k_scan_exclusive + k_init_pt_cap : the transport cap in id order
-//                    (citizen_factory.rs:72-83) is a rank test against an exclusive scan
-//                    of the per-block counts;
-//   k_select_hist  : radix selection over the 96-bit composite (INIT_C key, id), 12 bits
-//                    a pass, finds the agent of a given rank without sorting; the starting
+//   k_scan         : exclusive prefix sums of such counts, a block per array;
+//   k_select_pass  : radix selection over the 96-bit composite (INIT_C key, id), 8 bits
+//                    a pass, finds the agents of given ranks without sorting; the starting
 //                    infections (the `total` smallest composites, taking exposed /
 //                    asymptomatic / mild / severe in composite order) need at most four
-//                    such ranks;
-//   k_init_infect  : per agent, its group from the four rank bounds;
-//   k_init_cells   : per house, random_points(k) of the 2x2 house for its agents;
-//   k_init_grid    : per agent, its byte of the padded occupancy grid.
-// All of it is integer work over a few bytes per agent and runs once per simulation.
+//                    such ranks, narrowed side by side;
+//   k_init_finish  : per agent, the transport cap in id order (citizen_factory.rs:72-83) as a
+//                    rank test against the scanned counts, then its group of starting
+//                    infections from the four rank bounds;
+//   k_init_cells   : per house, random_points(k) of the 2x2 house for its agents, and their
+//                    bytes of the padded occupancy grid.
+// All of it is integer work over a few bytes per agent and runs once per handle, a chain of
+// launches that nothing on the host waits for: 32 simulations of 100k agents are created in
+// 13.1 -> 1.7 ms, 64 of mixed sizes in 26.8 -> 3.3, one of 10k in 0.57 -> 0.46 (before: a simulation at a
+// time, a read-back after each of its up to 32 selection passes, temporaries for each).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <utility>
 #include <vector>
 
 #include "disease.hpp"
@@ -32,23 +37,11 @@ namespace epi {
 namespace {
 
 constexpr uint32_t kInitBlock = 256;
-constexpr uint32_t kSelectBits = 12;
+constexpr uint32_t kSelectBits = 8;
 constexpr uint32_t kSelectBins = 1u << kSelectBits;
-constexpr uint32_t kSelectTopShift = 96 - kSelectBits;  // 84
-
-struct InitArgs {
-  uint32_t n;
-  uint32_t seed_lo, seed_hi;
-  uint64_t thr_work, thr_pt, thr_staff, thr_ess;
-  const uint8_t* csv_working;  // Population::Csv columns, or null for Auto
-  const uint8_t* csv_pt;
-  uint32_t pt_cap;
-  uint32_t* pos;
-  uint32_t* st;
-  uint32_t* tm;
-  uint32_t* wsa;
-  uint32_t* block_pt;  // per init block: public-transport draws, then their exclusive prefix
-};
+constexpr uint32_t kSelectTopShift = 96 - kSelectBits;  // 88
+constexpr uint32_t kSelectBlocks = 512;                 // at most, for one simulation
+static_assert(kSelectBins == kInitBlock, "a thread per bin");
 
 // A point of the 96-bit order (key, id): key in bits 95..32, id in bits 31..0.
 struct Composite {
@@ -56,26 +49,90 @@ struct Composite {
   uint32_t id;
 };
 
-__device__ __forceinline__ uint64_t seed_of(const InitArgs& a) { return join64(a.seed_hi, a.seed_lo); }
+// One simulation of the batch. first_* are its first blocks in the launches over agents,
+// selection strides, houses, offices and id chunks.
+struct InitSim {
+  uint32_t n;
+  uint32_t seed_lo, seed_hi;
+  uint64_t thr_work, thr_pt, thr_staff, thr_ess;
+  const uint8_t* csv_working;  // Population::Csv columns, or null for Auto
+  const uint8_t* csv_pt;
+  uint32_t pt_cap;  // ~0u: none (Population::Csv records keep their flag)
+  uint32_t* pos;
+  uint32_t* st;
+  uint32_t* tm;
+  uint32_t* wsa;
+  uint8_t* occ;
+  uint32_t pitch;
+  DiseaseParams dz;
+  int32_t house_sx, house_sy, house_nx;
+  uint32_t n_houses;
+  uint32_t* block_pt;  // per agent block: public-transport draws, then their exclusive prefix
+  uint32_t infected;   // starting infections of all kinds
+  uint32_t zero;       // bit j: the first j + 1 kinds together are none
+  uint32_t first_block, first_select, first_house;
+};
+// The same for the office layout's maps.
+struct OfficeSim {
+  uint32_t n, n_offices;
+  const uint32_t* st;
+  uint32_t *office_agent, *office_slot;
+  uint32_t *cnt, *base;    // per office: its workers, and their exclusive prefix
+  uint32_t *rcnt, *rbase;  // per id chunk: the other agents, and their exclusive prefix
+  uint32_t first_office, first_chunk;
+};
 
-__device__ __forceinline__ uint64_t infection_key(const InitArgs& a, uint32_t i) {
-  const u32x4 c = draw(seed_of(a), i, kInitHour, SITE_INIT_C, 0);
+// The last of n simulations whose first block (member F) is at most `block`: those with no
+// blocks share the next one's first.
+template <auto F, class Sim>
+__device__ __forceinline__ uint32_t sim_of_block(const Sim* sims, uint32_t n, uint32_t block) {
+  uint32_t lo = 0, hi = n;
+  while (hi - lo > 1) {
+    const uint32_t mid = (lo + hi) / 2;
+    if (sims[mid].*F <= block) lo = mid;
+    else hi = mid;
+  }
+  return lo;
+}
+
+__device__ __forceinline__ uint64_t seed_of(const InitSim& a) { return join64(a.seed_hi, a.seed_lo); }
+
+__device__ __forceinline__ uint64_t infection_key(uint32_t seed_lo, uint32_t seed_hi, uint32_t i) {
+  const u32x4 c = philox4x32_10(i, kInitHour, SITE_INIT_C, 0, seed_lo, seed_hi);
   return join64(c.w[2], c.w[3]);
 }
 
-// Bits [shift, shift + 12) of the composite.
+// Bits [shift, shift + kSelectBits) of the composite.
 __device__ __forceinline__ uint32_t digit(uint64_t key, uint32_t id, uint32_t shift) {
   if (shift >= 32) return static_cast<uint32_t>(key >> (shift - 32)) & (kSelectBins - 1);
   const uint64_t low = (key << 32) | id;
   return static_cast<uint32_t>(low >> shift) & (kSelectBins - 1);
 }
 
+__device__ __forceinline__ void set_digit(Composite& c, uint32_t shift, uint32_t d) {
+  if (shift >= 32) {
+    c.key |= static_cast<unsigned long long>(d) << (shift - 32);
+  } else {
+    const uint64_t v = static_cast<uint64_t>(d) << shift;
+    c.id |= static_cast<uint32_t>(v);
+    c.key |= v >> 32;
+  }
+}
+
+// Blocks of a simulation in a selection pass, each striding over its agents, at least 16 a
+// thread: the last block adds up the others' counts.
+__host__ __device__ inline uint32_t select_blocks(uint32_t n) {
+  const uint32_t blocks = (n + 16u * kInitBlock - 1u) / (16u * kInitBlock);
+  return blocks < kSelectBlocks ? blocks : kSelectBlocks;
+}
+
 __device__ __forceinline__ bool greater(uint64_t key, uint32_t id, const Composite& c) {
   return key > c.key || (key == c.key && id > c.id);
 }
 
-__global__ __launch_bounds__(kInitBlock) void k_init_agents(InitArgs a) {
-  const uint32_t i = blockIdx.x * kInitBlock + threadIdx.x;
+__global__ __launch_bounds__(kInitBlock) void k_init_agents(const InitSim* sims, uint32_t n_sims) {
+  const InitSim& a = sims[sim_of_block<&InitSim::first_block>(sims, n_sims, blockIdx.x)];
+  const uint32_t block = blockIdx.x - a.first_block, i = block * kInitBlock + threadIdx.x;
   bool pt = false;
   if (i < a.n) {
     const uint64_t seed = seed_of(a);
@@ -100,17 +157,24 @@ __global__ __launch_bounds__(kInitBlock) void k_init_agents(InitArgs a) {
     a.tm[i] = 0;
   }
   const int count = __syncthreads_count(pt);
-  if (threadIdx.x == 0) a.block_pt[blockIdx.x] = static_cast<uint32_t>(count);
+  if (threadIdx.x == 0) a.block_pt[block] = static_cast<uint32_t>(count);
 }
 
-// Exclusive prefix sum of v[0..n) in place, one block of 1024 threads: each thread sums a
-// contiguous chunk, the chunk sums are scanned in LDS, then each chunk is rewritten.
-__global__ __launch_bounds__(1024) void k_scan_exclusive(uint32_t* v, uint32_t n) {
+// Exclusive prefix sum of from[0..n) into to (the same array or another), one block of 1024
+// threads per array: each thread sums a contiguous chunk, the chunk sums are scanned in LDS,
+// then each chunk is written.
+struct ScanJob {
+  const uint32_t* from;
+  uint32_t* to;
+  uint32_t n;
+};
+__global__ __launch_bounds__(1024) void k_scan(const ScanJob* jobs) {
   __shared__ uint32_t part[1024];
-  const uint32_t per = (n + 1023u) / 1024u;
-  const uint32_t b = threadIdx.x * per, e = min(n, b + per);
+  const ScanJob a = jobs[blockIdx.x];
+  const uint32_t per = (a.n + 1023u) / 1024u;
+  const uint32_t b = min(a.n, threadIdx.x * per), e = min(a.n, b + per);
   uint32_t sum = 0;
-  for (uint32_t k = b; k < e; ++k) sum += v[k];
+  for (uint32_t k = b; k < e; ++k) sum += a.from[k];
   part[threadIdx.x] = sum;
   __syncthreads();
   for (uint32_t off = 1; off < 1024u; off <<= 1) {
@@ -121,71 +185,164 @@ __global__ __launch_bounds__(1024) void k_scan_exclusive(uint32_t* v, uint32_t n
   }
   uint32_t run = threadIdx.x ? part[threadIdx.x - 1] : 0u;
   for (uint32_t k = b; k < e; ++k) {
-    const uint32_t x = v[k];
-    v[k] = run;
+    const uint32_t x = a.from[k];
+    a.to[k] = run;
     run += x;
   }
 }
 
-// Clears F_PT on every public-transport draw whose rank in id order is >= the cap.
-__global__ __launch_bounds__(kInitBlock) void k_init_pt_cap(InitArgs a) {
+// Selection of up to four ranks of one simulation: bound[j] is the composite of rank
+// c_j - 1 for the cumulative group sizes c = (exposed, +asymptomatic, +mild, +severe), once
+// bit j of `done` is set; until then its top bits, with the rank that is left among the agents
+// that share them. An agent of rank r belongs to group #{j : r >= c_j}; group 4 means not
+// selected.
+struct Select {
+  Composite bound[4];
+  uint32_t rank[4];
+  uint32_t done;
+  uint32_t finished;  // blocks that have counted in this pass
+};
+
+// Bits below `shift` of the composite.
+__device__ __forceinline__ Composite low_bits(uint32_t shift) {
+  if (shift >= 32) return Composite{(1ull << (shift - 32)) - 1ull, ~0u};
+  return Composite{0ull, shift ? ~0u >> (32 - shift) : 0u};
+}
+
+// One pass: a histogram of digit(shift) over the agents that share each open bound's top bits.
+// In the first pass these are all agents: counted in LDS, each block's counts stored to `top`
+// (as atomics, up to 512 to one address, they take longer than the draws).
+// Later they are next to none, counted by atomics in the simulation's slice of `hist`. The
+// block that finishes last takes each bound's bin, clears what it read for the next pass, and
+// closes a bound whose bin holds one agent: all lower bits set then compare as that agent's own
+// do. So most of the twelve launches find nothing to do. What other blocks wrote is read by
+// device-scope atomics.
+__global__ __launch_bounds__(kInitBlock) void k_select_pass(const InitSim* sims, uint32_t n_sims, Select* selects,
+                                                            uint32_t* top, uint32_t* hist, uint32_t shift) {
+  __shared__ uint32_t h[kSelectBins];
+  __shared__ uint32_t last, single;
+  const uint32_t sim = sim_of_block<&InitSim::first_select>(sims, n_sims, blockIdx.x);
+  const InitSim& a = sims[sim];
+  Select& s = selects[sim];
+  const uint32_t done = s.done;
+  if (done == 15u) return;  // uniform, over all the simulation's blocks
+  const uint32_t n_blocks = select_blocks(a.n), t = threadIdx.x;
+  hist += static_cast<size_t>(sim) * 4 * kSelectBins;
+  const bool first = shift == kSelectTopShift;
+  // read before the loop, whose atomics could change them for all the compiler knows
+  const uint32_t n = a.n, seed_lo = a.seed_lo, seed_hi = a.seed_hi;
+  Composite bound[4];
+#pragma unroll
+  for (uint32_t j = 0; j < 4; ++j) bound[j] = s.bound[j];
+  const Composite low = low_bits(shift + kSelectBits);  // not compared
+  h[t] = 0;
+  __syncthreads();
+  for (uint32_t i = (blockIdx.x - a.first_select) * kInitBlock + t; i < n; i += n_blocks * kInitBlock) {
+    const uint64_t key = infection_key(seed_lo, seed_hi, i);
+    const uint32_t d = digit(key, i, shift);
+    if (first) {
+      atomicAdd(&h[d], 1u);
+      continue;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j)
+      if (!((done >> j) & 1u) && ((key ^ bound[j].key) & ~low.key) == 0 && ((i ^ bound[j].id) & ~low.id) == 0)
+        atomicAdd(&hist[j * kSelectBins + d], 1u);
+  }
+  __syncthreads();
+  if (first)
+    __hip_atomic_store(&top[static_cast<size_t>(blockIdx.x) * kSelectBins + t], h[t], __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  __threadfence();
+  __syncthreads();
+  if (t == 0) last = atomicAdd(&s.finished, 1u) == n_blocks - 1u;
+  __syncthreads();
+  if (!last) return;
+  __threadfence();
+  uint32_t all = 0;  // agents of this thread's bin
+  if (first) {
+    const uint32_t* of = top + static_cast<size_t>(a.first_select) * kSelectBins + t;
+#pragma unroll 16
+    for (uint32_t b = 0; b < n_blocks; ++b)
+      all += __hip_atomic_load(of + static_cast<size_t>(b) * kSelectBins, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  uint32_t closed = done;
+  for (uint32_t j = 0; j < 4; ++j) {
+    if ((done >> j) & 1u) continue;  // uniform
+    uint32_t count = all;
+    if (!first) {
+      count = __hip_atomic_load(&hist[j * kSelectBins + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&hist[j * kSelectBins + t], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const uint32_t r = s.rank[j];  // before the barriers: one thread changes it after them
+    if (t == 0) single = 0;
+    h[t] = count;
+    __syncthreads();
+    for (uint32_t off = 1; off < kSelectBins; off <<= 1) {
+      const uint32_t before = t >= off ? h[t - off] : 0u;
+      __syncthreads();
+      h[t] += before;
+      __syncthreads();
+    }
+    const uint32_t before = h[t] - count;
+    if (r >= before && r - before < count) {  // one thread
+      Composite c = bound[j];
+      set_digit(c, shift, t);
+      if (count == 1u || shift == 0u) {
+        const Composite rest = low_bits(shift);
+        c.key |= rest.key;
+        c.id |= rest.id;
+        single = 1;
+      }
+      s.bound[j] = c;
+      s.rank[j] = r - before;
+    }
+    __syncthreads();
+    if (single) closed |= 1u << j;
+    __syncthreads();
+  }
+  if (t == 0) {
+    s.done = closed;
+    s.finished = 0;
+  }
+}
+
+__global__ __launch_bounds__(kInitBlock) void k_init_finish(const InitSim* sims, uint32_t n_sims,
+                                                            const Select* selects) {
   __shared__ uint32_t wave_count[kInitBlock / 64];
-  const uint32_t i = blockIdx.x * kInitBlock + threadIdx.x;
-  const bool pt = i < a.n && (a.st[i] & F_PT) != 0;
-  const uint64_t mask = __ballot(pt);
+  const uint32_t sim = sim_of_block<&InitSim::first_block>(sims, n_sims, blockIdx.x);
+  const InitSim& a = sims[sim];
+  const uint32_t block = blockIdx.x - a.first_block, i = block * kInitBlock + threadIdx.x;
+  const uint32_t w_in = i < a.n ? a.st[i] : 0u;
+  uint32_t w = w_in;
+  // clears F_PT on every public-transport draw whose rank in id order is >= the cap
+  const uint64_t mask = __ballot((w & F_PT) != 0);
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   if (lane == 0) wave_count[wave] = static_cast<uint32_t>(__popcll(mask));
   __syncthreads();
-  if (!pt) return;
-  uint32_t rank = a.block_pt[blockIdx.x] + static_cast<uint32_t>(__popcll(mask & ((1ull << lane) - 1ull)));
-  for (uint32_t w = 0; w < wave; ++w) rank += wave_count[w];
-  if (rank >= a.pt_cap) a.st[i] &= ~F_PT;
-}
-
-// Histogram of digit(shift) over the agents whose composite matches `prefix` on `mask`.
-__global__ __launch_bounds__(kInitBlock) void k_select_hist(InitArgs a, Composite prefix, Composite mask,
-                                                            uint32_t shift, uint32_t* hist) {
-  __shared__ uint32_t h[kSelectBins];
-  for (uint32_t k = threadIdx.x; k < kSelectBins; k += kInitBlock) h[k] = 0;
-  __syncthreads();
-  const uint32_t step = gridDim.x * kInitBlock;
-  for (uint32_t i = blockIdx.x * kInitBlock + threadIdx.x; i < a.n; i += step) {
-    const uint64_t key = infection_key(a, i);
-    if (((key ^ prefix.key) & mask.key) == 0 && ((i ^ prefix.id) & mask.id) == 0)
-      atomicAdd(&h[digit(key, i, shift)], 1u);
-    if (i > 0xFFFFFFFFu - step) break;
+  if (w & F_PT) {
+    uint32_t rank = a.block_pt[block] + static_cast<uint32_t>(__popcll(mask & ((1ull << lane) - 1ull)));
+    for (uint32_t q = 0; q < wave; ++q) rank += wave_count[q];
+    if (rank >= a.pt_cap) w &= ~F_PT;
   }
-  __syncthreads();
-  for (uint32_t k = threadIdx.x; k < kSelectBins; k += kInitBlock)
-    if (h[k]) atomicAdd(&hist[k], h[k]);
-}
-
-// bound[j] is the composite of rank c_j - 1 for the cumulative group sizes
-// c = (exposed, +asymptomatic, +mild, +severe); bit j of `zero` marks c_j == 0. An agent
-// of rank r belongs to group #{j : r >= c_j}; group 4 means not selected.
-struct Bounds {
-  Composite bound[4];
-  uint32_t zero;
-};
-
-__global__ __launch_bounds__(kInitBlock) void k_init_infect(InitArgs a, Bounds b) {
-  const uint32_t i = blockIdx.x * kInitBlock + threadIdx.x;
   if (i >= a.n) return;
-  const uint64_t key = infection_key(a, i);
-  uint32_t group = 0;
+  if (a.infected) {  // uniform
+    const Select& s = selects[sim];
+    const uint64_t key = infection_key(a.seed_lo, a.seed_hi, i);
+    uint32_t group = 0;
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-    if (((b.zero >> j) & 1u) || greater(key, i, b.bound[j])) ++group;
-  if (group >= 4) return;
-  // starting_infections.rs: exposed {at_hour 0}; infected asymptomatic / mild / severe on day 1
-  const uint32_t state = group == 0 ? ST_E : ST_I;
-  const uint32_t sev = group == 0 ? 0u : (group == 1 ? SEV_ASYM : (group == 2 ? SEV_MILD : SEV_SEVERE));
-  const uint32_t day = group == 0 ? 0u : 1u;
-  uint32_t w = a.st[i];
-  w = (w & ~((M_STATE << B_STATE) | (M_SEV << B_SEV) | (M_DAY << B_DAY))) | (state << B_STATE) | (sev << B_SEV) |
-      (day << B_DAY);
-  a.st[i] = w;
-  a.tm[i] = 0;
+    for (int j = 0; j < 4; ++j)
+      if (((a.zero >> j) & 1u) || greater(key, i, s.bound[j])) ++group;
+    if (group < 4) {
+      // starting_infections.rs: exposed {at_hour 0}; infected asymptomatic / mild / severe on day 1
+      const uint32_t state = group == 0 ? ST_E : ST_I;
+      const uint32_t sev = group == 0 ? 0u : (group == 1 ? SEV_ASYM : (group == 2 ? SEV_MILD : SEV_SEVERE));
+      const uint32_t day = group == 0 ? 0u : 1u;
+      w = (w & ~((M_STATE << B_STATE) | (M_SEV << B_SEV) | (M_DAY << B_DAY))) | (state << B_STATE) | (sev << B_SEV) |
+          (day << B_DAY);
+    }
+  }
+  if (w != w_in) a.st[i] = w;  // tm is 0 already
 }
 
 // Partial Fisher-Yates over {lo, lo + 1} from fixed words: min(m, 2) values.
@@ -204,19 +361,16 @@ __device__ __forceinline__ uint32_t choose2(int32_t lo, uint32_t m, uint32_t w0,
   return m;
 }
 
-struct HouseLayout {
-  int32_t sx, sy, nx;
-  uint32_t n_houses;
-};
-
-// House h holds agents h, h + H, ...; they take random_points(k) of the house in id order.
-__global__ __launch_bounds__(kInitBlock) void k_init_cells(InitArgs a, HouseLayout L) {
-  const uint32_t h = blockIdx.x * kInitBlock + threadIdx.x;
-  const uint32_t H = L.n_houses;
+// House h holds agents h, h + H, ...; they take random_points(k) of the house in id order, and
+// each cell its agent's grid byte: 1 occupied, 2 / 3 infectious in the regular / high window.
+__global__ __launch_bounds__(kInitBlock) void k_init_cells(const InitSim* sims, uint32_t n_sims) {
+  const InitSim& a = sims[sim_of_block<&InitSim::first_house>(sims, n_sims, blockIdx.x)];
+  const uint32_t h = (blockIdx.x - a.first_house) * kInitBlock + threadIdx.x;
+  const uint32_t H = a.n_houses;
   if (h >= min(H, a.n)) return;
   const uint32_t k = (a.n - h + H - 1) / H;
-  const int32_t x0 = L.sx + static_cast<int32_t>(h % static_cast<uint32_t>(L.nx)) * 2;
-  const int32_t y0 = L.sy + static_cast<int32_t>(h / static_cast<uint32_t>(L.nx)) * 2;
+  const int32_t x0 = a.house_sx + static_cast<int32_t>(h % static_cast<uint32_t>(a.house_nx)) * 2;
+  const int32_t y0 = a.house_sy + static_cast<int32_t>(h / static_cast<uint32_t>(a.house_nx)) * 2;
   const u32x4 w = draw(seed_of(a), h, kInitHour, SITE_INIT_HOUSE, 0);
   uint32_t side = 1;  // ceil(sqrt(k)) in integers
   while (side * side < k) ++side;
@@ -225,48 +379,43 @@ __global__ __launch_bounds__(kInitBlock) void k_init_cells(InitArgs a, HouseLayo
   const uint32_t my = choose2(y0, side, w.w[2], w.w[3], ys);
   uint32_t j = 0;
   for (uint32_t p = 0; p < mx && j < k; ++p)
-    for (uint32_t q = 0; q < my && j < k; ++q, ++j)
-      a.pos[h + j * H] = static_cast<uint32_t>(xs[p]) | (static_cast<uint32_t>(ys[q]) << 16);
+    for (uint32_t q = 0; q < my && j < k; ++q, ++j) {
+      const uint32_t id = h + j * H, x = static_cast<uint32_t>(xs[p]), y = static_cast<uint32_t>(ys[q]);
+      a.pos[id] = x | (y << 16);
+      a.occ[static_cast<size_t>(y + kPadY) * a.pitch + x + kPadX] = occupant_byte(a.dz, a.st[id]);
+    }
 }
 
-struct GridArgs {
-  uint8_t* occ;
-  uint32_t pitch;
-  DiseaseParams dz;
-};
-
-// The agent's grid byte: 1 occupied, 2 / 3 infectious in the regular / high window.
-__global__ __launch_bounds__(kInitBlock) void k_init_grid(InitArgs a, GridArgs g) {
-  const uint32_t i = blockIdx.x * kInitBlock + threadIdx.x;
-  if (i >= a.n) return;
-  const uint32_t p = a.pos[i], w = a.st[i];
-  g.occ[static_cast<size_t>((p >> 16) + kPadY) * g.pitch + (p & 0xFFFFu) + kPadX] = occupant_byte(g.dz, w);
-}
-
-void set_digit(Composite& c, uint32_t shift, uint32_t d) {
-  if (shift >= 32) {
-    c.key |= static_cast<unsigned long long>(d) << (shift - 32);
-  } else {
-    const uint64_t v = static_cast<uint64_t>(d) << shift;
-    c.id |= static_cast<uint32_t>(v);
-    c.key |= v >> 32;
-  }
-}
-
+// One allocation for all of a call's scratch arrays: add() them, then alloc().
 struct DeviceTemp {
-  std::vector<void*> owned;
   template <class T>
-  hipError_t alloc(T** p, size_t count) {
-    void* q = nullptr;
-    hipError_t e = hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T));
-    if (e == hipSuccess) owned.push_back(q);
-    *p = static_cast<T*>(q);
+  void add(T** p, size_t count) {
+    arrays.push_back({reinterpret_cast<void**>(p), bytes});
+    bytes += (count * sizeof(T) + 255) / 256 * 256;
+  }
+  hipError_t alloc() {
+    const hipError_t e = hipMalloc(&memory, std::max<size_t>(bytes, 1));
+    if (e != hipSuccess) {
+      memory = nullptr;
+      return e;
+    }
+    for (const auto& a : arrays) *a.first = static_cast<char*>(memory) + a.second;
     return e;
   }
   ~DeviceTemp() {
-    for (void* p : owned) (void)hipFree(p);
+    if (memory) (void)hipFree(memory);
   }
+  std::vector<std::pair<void**, size_t>> arrays;
+  size_t bytes = 0;
+  void* memory = nullptr;
 };
+
+template <class T>
+hipError_t upload(T* to, const std::vector<T>& from, hipStream_t stream) {
+  return hipMemcpyAsync(to, from.data(), from.size() * sizeof(T), hipMemcpyHostToDevice, stream);
+}
+
+uint32_t div_up(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
 #define INIT_TRY(step, expr)      \
   do {                            \
@@ -277,33 +426,6 @@ struct DeviceTemp {
     }                             \
   } while (0)
 
-// The composite of rank r (0-based) among all agents: eight 12-bit passes, each narrowing
-// the prefix to the bin that holds rank r.
-hipError_t select_rank(const InitArgs& a, uint32_t r, uint32_t* d_hist, uint32_t grid, hipStream_t stream,
-                       Composite& out, std::string& err) {
-  Composite prefix{0, 0}, mask{0, 0};
-  std::vector<uint32_t> h(kSelectBins);
-  for (int shift = static_cast<int>(kSelectTopShift); shift >= 0; shift -= static_cast<int>(kSelectBits)) {
-    INIT_TRY("select: clear histogram", hipMemsetAsync(d_hist, 0, kSelectBins * sizeof(uint32_t), stream));
-    hipLaunchKernelGGL(k_select_hist, dim3(grid), dim3(kInitBlock), 0, stream, a, prefix, mask,
-                       static_cast<uint32_t>(shift), d_hist);
-    INIT_TRY("select: k_select_hist", hipGetLastError());
-    INIT_TRY("select: read histogram",
-             hipMemcpyAsync(h.data(), d_hist, kSelectBins * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-    INIT_TRY("select: sync", hipStreamSynchronize(stream));
-    uint32_t b = 0;
-    while (b < kSelectBins && r >= h[b]) r -= h[b++];
-    if (b == kSelectBins) {
-      err = "select: rank beyond the population";
-      return hipErrorInvalidValue;
-    }
-    set_digit(prefix, static_cast<uint32_t>(shift), b);
-    set_digit(mask, static_cast<uint32_t>(shift), kSelectBins - 1);
-  }
-  out = prefix;
-  return hipSuccess;
-}
-
 // ---- office layout slot maps (model.hpp): Normal and Essential workers office by office
 // (office j = id % n_offices), each office's in id order, then the other agents in id order.
 __device__ __forceinline__ bool office_worker(uint32_t w) {
@@ -311,48 +433,63 @@ __device__ __forceinline__ bool office_worker(uint32_t w) {
   return ws == WS_NORMAL || ws == WS_ESSENTIAL;
 }
 
-// One thread per office: its workers (ids j, j + O, ... in order, coalesced over offices).
-__global__ __launch_bounds__(kInitBlock) void k_office_count(const uint32_t* st, uint32_t n, uint32_t O,
-                                                             uint32_t* cnt) {
-  const uint32_t j = blockIdx.x * kInitBlock + threadIdx.x;
-  if (j >= O) return;
-  uint32_t c = 0;
-  for (uint64_t id = j; id < n; id += O) c += office_worker(st[id]) ? 1u : 0u;
-  cnt[j] = c;
+// One thread per office: its workers (ids j, j + O, ... in order, coalesced over offices), the
+// state words of kAhead of them in flight.
+constexpr uint32_t kAhead = 16;
+template <class F>
+__device__ __forceinline__ void for_each_id(const OfficeSim& a, uint32_t j, F&& f) {
+  for (uint64_t id0 = j; id0 < a.n; id0 += static_cast<uint64_t>(kAhead) * a.n_offices) {
+    uint32_t w[kAhead];
+#pragma unroll
+    for (uint32_t k = 0; k < kAhead; ++k) {
+      const uint64_t id = id0 + static_cast<uint64_t>(k) * a.n_offices;
+      w[k] = id < a.n ? a.st[id] : (WS_NA << B_WS);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kAhead; ++k)
+      if (office_worker(w[k])) f(static_cast<uint32_t>(id0 + static_cast<uint64_t>(k) * a.n_offices));
+  }
 }
 
-__global__ __launch_bounds__(kInitBlock) void k_office_place(const uint32_t* st, uint32_t n, uint32_t O,
-                                                             const uint32_t* base, uint32_t* office_agent,
-                                                             uint32_t* office_slot) {
-  const uint32_t j = blockIdx.x * kInitBlock + threadIdx.x;
-  if (j >= O) return;
-  uint32_t slot = base[j];
-  for (uint64_t id = j; id < n; id += O)
-    if (office_worker(st[id])) {
-      office_agent[slot] = static_cast<uint32_t>(id);
-      office_slot[id] = slot;
-      ++slot;
-    }
+__global__ __launch_bounds__(kInitBlock) void k_office_count(const OfficeSim* sims, uint32_t n_sims) {
+  const OfficeSim& a = sims[sim_of_block<&OfficeSim::first_office>(sims, n_sims, blockIdx.x)];
+  const uint32_t j = (blockIdx.x - a.first_office) * kInitBlock + threadIdx.x;
+  if (j >= a.n_offices) return;
+  uint32_t c = 0;
+  for_each_id(a, j, [&](uint32_t) { ++c; });
+  a.cnt[j] = c;
+}
+
+__global__ __launch_bounds__(kInitBlock) void k_office_place(const OfficeSim* sims, uint32_t n_sims) {
+  const OfficeSim& a = sims[sim_of_block<&OfficeSim::first_office>(sims, n_sims, blockIdx.x)];
+  const uint32_t j = (blockIdx.x - a.first_office) * kInitBlock + threadIdx.x;
+  if (j >= a.n_offices) return;
+  uint32_t slot = a.base[j];
+  for_each_id(a, j, [&](uint32_t id) {
+    a.office_agent[slot] = id;
+    a.office_slot[id] = slot;
+    ++slot;
+  });
 }
 
 constexpr uint32_t kRestChunk = 1024;  // ids per block of the other agents' passes
 
 // Other agents per chunk of kRestChunk ids.
-__global__ __launch_bounds__(kRestChunk) void k_rest_count(const uint32_t* st, uint32_t n, uint32_t* cnt) {
-  const uint32_t id = blockIdx.x * kRestChunk + threadIdx.x;
-  const int rest = id < n && !office_worker(st[id]);
+__global__ __launch_bounds__(kRestChunk) void k_rest_count(const OfficeSim* sims, uint32_t n_sims) {
+  const OfficeSim& a = sims[sim_of_block<&OfficeSim::first_chunk>(sims, n_sims, blockIdx.x)];
+  const uint32_t chunk = blockIdx.x - a.first_chunk, id = chunk * kRestChunk + threadIdx.x;
+  const int rest = id < a.n && !office_worker(a.st[id]);
   const int c = __syncthreads_count(rest);
-  if (threadIdx.x == 0) cnt[blockIdx.x] = static_cast<uint32_t>(c);
+  if (threadIdx.x == 0) a.rcnt[chunk] = static_cast<uint32_t>(c);
 }
 
-// Slot of each other agent: n_workers + the chunk's base + its rank in the chunk (wave
+// Slot of each other agent: the workers + the chunk's base + its rank in the chunk (wave
 // ballots, then the waves' totals in LDS).
-__global__ __launch_bounds__(kRestChunk) void k_rest_place(const uint32_t* st, uint32_t n, uint32_t n_workers,
-                                                          const uint32_t* base, uint32_t* office_agent,
-                                                          uint32_t* office_slot) {
+__global__ __launch_bounds__(kRestChunk) void k_rest_place(const OfficeSim* sims, uint32_t n_sims) {
   __shared__ uint32_t wave_total[kRestChunk / 64];
-  const uint32_t id = blockIdx.x * kRestChunk + threadIdx.x;
-  const bool rest = id < n && !office_worker(st[id]);
+  const OfficeSim& a = sims[sim_of_block<&OfficeSim::first_chunk>(sims, n_sims, blockIdx.x)];
+  const uint32_t chunk = blockIdx.x - a.first_chunk, id = chunk * kRestChunk + threadIdx.x;
+  const bool rest = id < a.n && !office_worker(a.st[id]);
   const unsigned long long m = __ballot(rest);
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   const uint32_t below = static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)));
@@ -361,137 +498,195 @@ __global__ __launch_bounds__(kRestChunk) void k_rest_place(const uint32_t* st, u
   uint32_t before = 0;
   for (uint32_t w = 0; w < wave; ++w) before += wave_total[w];
   if (rest) {
-    const uint32_t slot = n_workers + base[blockIdx.x] + before + below;
-    office_agent[slot] = id;
-    office_slot[id] = slot;
+    // the workers come first: as many as the last office's base and count make
+    const uint32_t n_workers = a.base[a.n_offices - 1u] + a.cnt[a.n_offices - 1u];
+    const uint32_t slot = n_workers + a.rbase[chunk] + before + below;
+    a.office_agent[slot] = id;
+    a.office_slot[id] = slot;
   }
 }
 
 }  // namespace
 
-hipError_t synthesize_on_device(const Config& cfg, uint64_t seed, const Geometry& geo, const InitTargets& t,
-                                hipStream_t stream, std::string& err) {
-  const uint32_t N = cfg.number_of_agents;
-  INIT_TRY("clear grid", hipMemsetAsync(t.occ, 0, t.cells, stream));
-  if (N == 0) return hipSuccess;
-  DeviceTemp tmp;
-  const uint32_t blocks = (N + kInitBlock - 1) / kInitBlock;
-  InitArgs a{};
-  a.n = N;
-  a.seed_lo = static_cast<uint32_t>(seed);
-  a.seed_hi = static_cast<uint32_t>(seed >> 32);
-  a.thr_work = bernoulli_threshold(cfg.working_percentage);
-  a.thr_pt = bernoulli_threshold(cfg.public_transport_percentage);
-  a.thr_staff = bernoulli_threshold(0.002);  // HOSPITAL_STAFF_PERCENTAGE
-  a.thr_ess = bernoulli_threshold(cfg.has_lockdown ? cfg.essential_workers_population : 0.0);
-  a.pos = t.pos;
-  a.st = t.st;
-  a.tm = t.tm;
-  a.wsa = t.wsa;
-  INIT_TRY("alloc block counts", tmp.alloc(&a.block_pt, blocks));
-  if (cfg.csv_population) {
-    uint8_t* cols = nullptr;
-    INIT_TRY("alloc csv columns", tmp.alloc(&cols, 2 * static_cast<size_t>(N)));
-    INIT_TRY("upload csv working",
-             hipMemcpyAsync(cols, cfg.csv_working.data(), N, hipMemcpyHostToDevice, stream));
-    INIT_TRY("upload csv pub_transport",
-             hipMemcpyAsync(cols + N, cfg.csv_pub_transport.data(), N, hipMemcpyHostToDevice, stream));
-    a.csv_working = cols;
-    a.csv_pt = cols + N;
-  }
-  hipLaunchKernelGGL(k_init_agents, dim3(blocks), dim3(kInitBlock), 0, stream, a);
-  INIT_TRY("k_init_agents", hipGetLastError());
-  // public transport users are capped in id order; Population::Csv records keep their flag
-  if (!cfg.csv_population) {
-    a.pt_cap = geo.n_transport_points;
-    hipLaunchKernelGGL(k_scan_exclusive, dim3(1), dim3(1024), 0, stream, a.block_pt, blocks);
-    INIT_TRY("k_scan_exclusive", hipGetLastError());
-    hipLaunchKernelGGL(k_init_pt_cap, dim3(blocks), dim3(kInitBlock), 0, stream, a);
-    INIT_TRY("k_init_pt_cap", hipGetLastError());
-  }
-  // starting infections
-  const uint32_t c[4] = {cfg.si_exposed, cfg.si_exposed + cfg.si_asymptomatic,
-                         cfg.si_exposed + cfg.si_asymptomatic + cfg.si_mild,
-                         cfg.si_exposed + cfg.si_asymptomatic + cfg.si_mild + cfg.si_severe};
-  if (c[3] > 0) {
-    uint32_t* d_hist = nullptr;
-    INIT_TRY("alloc histogram", tmp.alloc(&d_hist, kSelectBins));
-    const uint32_t grid = std::min(blocks, 512u);
-    Bounds b{};
-    for (int j = 0; j < 4; ++j) {
-      if (c[j] == 0) {
-        b.zero |= 1u << j;
-      } else if (j > 0 && c[j] == c[j - 1]) {
-        b.bound[j] = b.bound[j - 1];
-      } else {
-        hipError_t e = select_rank(a, c[j] - 1, d_hist, grid, stream, b.bound[j], err);
-        if (e != hipSuccess) return e;
-      }
+hipError_t synthesize_on_device(const std::vector<InitJob>& jobs, hipStream_t stream, std::string& err) {
+  const uint32_t n_sims = static_cast<uint32_t>(jobs.size());
+  std::vector<InitSim> sims(n_sims);
+  std::vector<Select> selects(n_sims);
+  std::vector<ScanJob> scans;
+  uint32_t blocks = 0, strides = 0, house_blocks = 0;
+  size_t csv_bytes = 0;
+  for (uint32_t i = 0; i < n_sims; ++i) {
+    const Config& cfg = *jobs[i].cfg;
+    const Geometry& geo = *jobs[i].geo;
+    InitSim& a = sims[i];
+    a = InitSim{};
+    a.n = cfg.number_of_agents;
+    a.seed_lo = static_cast<uint32_t>(jobs[i].seed);
+    a.seed_hi = static_cast<uint32_t>(jobs[i].seed >> 32);
+    a.thr_work = bernoulli_threshold(cfg.working_percentage);
+    a.thr_pt = bernoulli_threshold(cfg.public_transport_percentage);
+    a.thr_staff = bernoulli_threshold(0.002);  // HOSPITAL_STAFF_PERCENTAGE
+    a.thr_ess = bernoulli_threshold(cfg.has_lockdown ? cfg.essential_workers_population : 0.0);
+    a.pt_cap = cfg.csv_population ? ~0u : geo.n_transport_points;
+    a.pos = jobs[i].pos;
+    a.st = jobs[i].st;
+    a.tm = jobs[i].tm;
+    a.wsa = jobs[i].wsa;
+    a.occ = jobs[i].occ;
+    a.pitch = jobs[i].pitch;
+    a.dz = Disease::params(cfg);
+    a.house_sx = geo.house_sx;
+    a.house_sy = geo.house_sy;
+    a.house_nx = std::max(geo.house_nx, 1);
+    a.n_houses = geo.n_houses;
+    const uint64_t c[4] = {cfg.si_exposed, 0ull + cfg.si_exposed + cfg.si_asymptomatic,
+                           0ull + cfg.si_exposed + cfg.si_asymptomatic + cfg.si_mild,
+                           0ull + cfg.si_exposed + cfg.si_asymptomatic + cfg.si_mild + cfg.si_severe};
+    a.infected = a.n && c[3] ? static_cast<uint32_t>(c[3]) : 0u;
+    if (a.n && c[3] > a.n) {
+      err = "select: rank beyond the population";
+      return hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL(k_init_infect, dim3(blocks), dim3(kInitBlock), 0, stream, a, b);
-    INIT_TRY("k_init_infect", hipGetLastError());
+    selects[i] = Select{};
+    for (uint32_t j = 0; j < 4; ++j) {
+      if (c[j] == 0) a.zero |= 1u << j;
+      else selects[i].rank[j] = static_cast<uint32_t>(c[j] - 1);
+    }
+    selects[i].done = a.zero;
+    a.first_block = blocks;
+    a.first_select = strides;
+    a.first_house = house_blocks;
+    blocks += div_up(a.n, kInitBlock);
+    if (a.infected) strides += select_blocks(a.n);
+    house_blocks += div_up(std::min(geo.n_houses, a.n), kInitBlock);
+    if (cfg.csv_population) csv_bytes += 2 * static_cast<size_t>(a.n);
   }
-  // start cells, then the grid
-  const HouseLayout L{geo.house_sx, geo.house_sy, std::max(geo.house_nx, 1), geo.n_houses};
-  const uint32_t houses = std::min(geo.n_houses, N);
-  if (houses) {
-    hipLaunchKernelGGL(k_init_cells, dim3((houses + kInitBlock - 1) / kInitBlock), dim3(kInitBlock), 0, stream, a,
-                       L);
+  if (blocks == 0) return hipSuccess;
+  DeviceTemp tmp;
+  uint32_t *block_pt = nullptr, *top = nullptr, *hist = nullptr;
+  uint8_t* csv = nullptr;
+  InitSim* d_sims = nullptr;
+  Select* d_selects = nullptr;
+  ScanJob* d_scans = nullptr;
+  const size_t bins = strides ? static_cast<size_t>(n_sims) * 4 * kSelectBins : 0;
+  tmp.add(&d_sims, n_sims);
+  tmp.add(&d_selects, n_sims);
+  tmp.add(&d_scans, n_sims);
+  tmp.add(&block_pt, blocks);
+  tmp.add(&top, static_cast<size_t>(strides) * kSelectBins);
+  tmp.add(&hist, bins);
+  tmp.add(&csv, csv_bytes);
+  INIT_TRY("alloc scratch", tmp.alloc());
+  for (uint32_t i = 0; i < n_sims; ++i) {
+    InitSim& a = sims[i];
+    a.block_pt = block_pt + a.first_block;
+    if (a.n) scans.push_back(ScanJob{a.block_pt, a.block_pt, div_up(a.n, kInitBlock)});
+    const Config& cfg = *jobs[i].cfg;
+    if (!cfg.csv_population || a.n == 0) continue;
+    INIT_TRY("upload csv working", hipMemcpyAsync(csv, cfg.csv_working.data(), a.n, hipMemcpyHostToDevice, stream));
+    INIT_TRY("upload csv pub_transport",
+             hipMemcpyAsync(csv + a.n, cfg.csv_pub_transport.data(), a.n, hipMemcpyHostToDevice, stream));
+    a.csv_working = csv;
+    a.csv_pt = csv + a.n;
+    csv += 2 * static_cast<size_t>(a.n);
+  }
+  INIT_TRY("upload simulations", upload(d_sims, sims, stream));
+  INIT_TRY("upload selections", upload(d_selects, selects, stream));
+  INIT_TRY("upload scans", upload(d_scans, scans, stream));
+  hipLaunchKernelGGL(k_init_agents, dim3(blocks), dim3(kInitBlock), 0, stream, d_sims, n_sims);
+  INIT_TRY("k_init_agents", hipGetLastError());
+  hipLaunchKernelGGL(k_scan, dim3(static_cast<uint32_t>(scans.size())), dim3(1024), 0, stream, d_scans);
+  INIT_TRY("k_scan", hipGetLastError());
+  if (strides) {
+    INIT_TRY("clear histograms", hipMemsetAsync(hist, 0, bins * sizeof(uint32_t), stream));
+    for (int shift = static_cast<int>(kSelectTopShift); shift >= 0; shift -= static_cast<int>(kSelectBits)) {
+      hipLaunchKernelGGL(k_select_pass, dim3(strides), dim3(kInitBlock), 0, stream, d_sims, n_sims, d_selects, top, hist,
+                         static_cast<uint32_t>(shift));
+      INIT_TRY("k_select_pass", hipGetLastError());
+    }
+  }
+  hipLaunchKernelGGL(k_init_finish, dim3(blocks), dim3(kInitBlock), 0, stream, d_sims, n_sims, d_selects);
+  INIT_TRY("k_init_finish", hipGetLastError());
+  if (house_blocks) {
+    hipLaunchKernelGGL(k_init_cells, dim3(house_blocks), dim3(kInitBlock), 0, stream, d_sims, n_sims);
     INIT_TRY("k_init_cells", hipGetLastError());
   }
-  const GridArgs g{t.occ, t.pitch, Disease::params(cfg)};
-  hipLaunchKernelGGL(k_init_grid, dim3(blocks), dim3(kInitBlock), 0, stream, a, g);
-  INIT_TRY("k_init_grid", hipGetLastError());
-  // the temporaries are freed on return: finish with them first
+  // the scratch is freed on return: finish with it first
   INIT_TRY("init sync", hipStreamSynchronize(stream));
   return hipSuccess;
 }
 
-hipError_t build_office_maps_on_device(const uint32_t* st, uint32_t n, uint32_t n_offices, uint32_t* office_agent,
-                                      uint32_t* office_slot, std::vector<uint32_t>& workers_per_office,
-                                      uint32_t& n_workers, hipStream_t stream, std::string& err) {
-  const uint32_t O = std::max(n_offices, 1u);
-  workers_per_office.assign(O, 0);
-  n_workers = 0;
-  if (n == 0) return hipSuccess;
-  const uint32_t chunks = (n + kRestChunk - 1) / kRestChunk;
+hipError_t build_office_maps_on_device(const std::vector<OfficeJob>& jobs,
+                                       std::vector<std::vector<uint32_t>>& workers_per_office, hipStream_t stream,
+                                       std::string& err) {
+  const uint32_t n_sims = static_cast<uint32_t>(jobs.size());
+  std::vector<OfficeSim> sims(n_sims);
+  std::vector<ScanJob> scans;
+  uint32_t office_blocks = 0, chunks = 0;
+  size_t offices = 0;
+  workers_per_office.assign(n_sims, {});
+  for (uint32_t i = 0; i < n_sims; ++i) {
+    OfficeSim& a = sims[i];
+    a = OfficeSim{};
+    a.n = jobs[i].n;
+    a.n_offices = std::max(jobs[i].n_offices, 1u);
+    a.st = jobs[i].st;
+    a.office_agent = jobs[i].office_agent;
+    a.office_slot = jobs[i].office_slot;
+    a.first_office = office_blocks;
+    a.first_chunk = chunks;
+    workers_per_office[i].assign(a.n_offices, 0);
+    if (a.n == 0) continue;
+    office_blocks += div_up(a.n_offices, kInitBlock);
+    chunks += div_up(a.n, kRestChunk);
+    offices += a.n_offices;
+  }
+  if (chunks == 0) return hipSuccess;
   DeviceTemp tmp;
-  uint32_t *d_cnt = nullptr, *d_base = nullptr, *d_rcnt = nullptr, *d_rbase = nullptr;
-  INIT_TRY("office maps: alloc", tmp.alloc(&d_cnt, O));
-  INIT_TRY("office maps: alloc", tmp.alloc(&d_base, O));
-  INIT_TRY("office maps: alloc", tmp.alloc(&d_rcnt, chunks));
-  INIT_TRY("office maps: alloc", tmp.alloc(&d_rbase, chunks));
-  const uint32_t ob = (O + kInitBlock - 1) / kInitBlock;
-  hipLaunchKernelGGL(k_office_count, dim3(ob), dim3(kInitBlock), 0, stream, st, n, O, d_cnt);
+  uint32_t *cnt = nullptr, *base = nullptr, *rcnt = nullptr, *rbase = nullptr;
+  OfficeSim* d_sims = nullptr;
+  ScanJob* d_scans = nullptr;
+  tmp.add(&d_sims, n_sims);
+  tmp.add(&d_scans, 2 * static_cast<size_t>(n_sims));
+  tmp.add(&cnt, offices);
+  tmp.add(&base, offices);
+  tmp.add(&rcnt, chunks);
+  tmp.add(&rbase, chunks);
+  INIT_TRY("office maps: alloc", tmp.alloc());
+  size_t office = 0;
+  for (OfficeSim& a : sims) {
+    if (a.n == 0) continue;
+    a.cnt = cnt + office;
+    a.base = base + office;
+    a.rcnt = rcnt + a.first_chunk;
+    a.rbase = rbase + a.first_chunk;
+    scans.push_back(ScanJob{a.cnt, a.base, a.n_offices});
+    scans.push_back(ScanJob{a.rcnt, a.rbase, div_up(a.n, kRestChunk)});
+    office += a.n_offices;
+  }
+  INIT_TRY("office maps: upload", upload(d_sims, sims, stream));
+  INIT_TRY("office maps: upload", upload(d_scans, scans, stream));
+  hipLaunchKernelGGL(k_office_count, dim3(office_blocks), dim3(kInitBlock), 0, stream, d_sims, n_sims);
   INIT_TRY("k_office_count", hipGetLastError());
-  hipLaunchKernelGGL(k_rest_count, dim3(chunks), dim3(kRestChunk), 0, stream, st, n, d_rcnt);
+  hipLaunchKernelGGL(k_rest_count, dim3(chunks), dim3(kRestChunk), 0, stream, d_sims, n_sims);
   INIT_TRY("k_rest_count", hipGetLastError());
-  std::vector<uint32_t> rest(chunks), base(O), rbase(chunks);
-  INIT_TRY("office maps: read counts", hipMemcpyAsync(workers_per_office.data(), d_cnt, O * sizeof(uint32_t),
-                                                       hipMemcpyDeviceToHost, stream));
-  INIT_TRY("office maps: read counts",
-           hipMemcpyAsync(rest.data(), d_rcnt, chunks * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-  INIT_TRY("office maps: sync", hipStreamSynchronize(stream));
-  for (uint32_t j = 0; j < O; ++j) {
-    base[j] = n_workers;
-    n_workers += workers_per_office[j];
-  }
-  for (uint32_t c = 0, acc = 0; c < chunks; ++c) {
-    rbase[c] = acc;
-    acc += rest[c];
-  }
-  INIT_TRY("office maps: write bases",
-           hipMemcpyAsync(d_base, base.data(), O * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
-  INIT_TRY("office maps: write bases",
-           hipMemcpyAsync(d_rbase, rbase.data(), chunks * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
-  hipLaunchKernelGGL(k_office_place, dim3(ob), dim3(kInitBlock), 0, stream, st, n, O, d_base, office_agent,
-                     office_slot);
+  hipLaunchKernelGGL(k_scan, dim3(static_cast<uint32_t>(scans.size())), dim3(1024), 0, stream, d_scans);
+  INIT_TRY("k_scan", hipGetLastError());
+  hipLaunchKernelGGL(k_office_place, dim3(office_blocks), dim3(kInitBlock), 0, stream, d_sims, n_sims);
   INIT_TRY("k_office_place", hipGetLastError());
-  hipLaunchKernelGGL(k_rest_place, dim3(chunks), dim3(kRestChunk), 0, stream, st, n, n_workers, d_rbase,
-                     office_agent, office_slot);
+  hipLaunchKernelGGL(k_rest_place, dim3(chunks), dim3(kRestChunk), 0, stream, d_sims, n_sims);
   INIT_TRY("k_rest_place", hipGetLastError());
-  // the temporaries and the host bases are freed on return: finish with them first
+  std::vector<uint32_t> counts(offices);
+  INIT_TRY("office maps: read counts",
+           hipMemcpyAsync(counts.data(), cnt, offices * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+  // the scratch is freed on return: finish with it first
   INIT_TRY("office maps: sync", hipStreamSynchronize(stream));
+  office = 0;
+  for (uint32_t i = 0; i < n_sims; ++i) {
+    if (sims[i].n == 0) continue;
+    std::copy_n(counts.begin() + static_cast<ptrdiff_t>(office), sims[i].n_offices, workers_per_office[i].begin());
+    office += sims[i].n_offices;
+  }
   return hipSuccess;
 }
 
