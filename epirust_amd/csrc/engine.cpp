@@ -782,12 +782,10 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
     event_off += D.event_cap;
     s->max_hour = std::max(s->max_hour, c.hours > 1 ? c.hours - 1 : 0u);
     std::memcpy(&s->counts0[7 * i], pops[i].counts0, sizeof(pops[i].counts0));
-    const auto cells = [](const Rect& r) {
-      return static_cast<uint32_t>(r.x1 - r.x0 + 1) * static_cast<uint32_t>(r.y1 - r.y0 + 1);
-    };
-    const uint32_t hosp_cells = std::max(cells(G.hosp0), cells(G.hosp1));
-    const uint32_t per_block = s->shape.hosp_block * s->shape.hosp_cells_per_thread;
-    for (uint32_t first = 0; first < hosp_cells; first += per_block)
+    const auto items = [](const Rect& r) { return hospital_items(r) * static_cast<uint32_t>(r.y1 - r.y0 + 1); };
+    const uint32_t hosp_items = std::max(items(G.hosp0), items(G.hosp1));
+    const uint32_t per_block = s->shape.hosp_block * s->shape.hosp_items_per_thread;
+    for (uint32_t first = 0; first < hosp_items; first += per_block)
       s->hosp_blocks.push_back(BlockRef{i, first});
   }
   s->n_agents = agent_off;

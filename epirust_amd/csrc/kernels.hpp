@@ -24,7 +24,7 @@ struct DevView {
   const AgentBlock* agent_blocks;  // per agent block; the office view has its own table
   const uint32_t* office_agent;    // office view: slot -> agent id (per simulation from agent_off)
   const uint32_t* office_slot;     // office view: agent id -> slot
-  const BlockRef* hosp_blocks;   // per hospital-scan block: (sim, first cell)
+  const BlockRef* hosp_blocks;   // per hospital-scan block: (sim, first item)
   Counts7* rows;
   Event* events;
   const uint32_t* vacc_hour;
@@ -49,7 +49,7 @@ struct LaunchShape {
   uint32_t agent_blocks = 0;     // total agent blocks over the batch (home layout)
   uint32_t office_agent_blocks = 0;  // the same for the office layout's table
   uint32_t hosp_block = 256;     // threads per hospital-scan block
-  uint32_t hosp_cells_per_thread = 8;
+  uint32_t hosp_items_per_thread = 2;
   uint32_t hosp_blocks = 0;
   uint32_t n_sims = 0;
 };

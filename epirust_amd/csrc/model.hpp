@@ -155,7 +155,13 @@ struct alignas(64) SimState {
   uint64_t night_vacc_thr;
 };
 
-// Launch-table entry: (simulation, first hospital cell).
+// The hospital scan's items: 16 cells of a row, from the aligned word of its first cell on.
+constexpr uint32_t kHospitalItem = 16;
+inline constexpr uint32_t hospital_items(const Rect& r) {  // of one row
+  return (static_cast<uint32_t>(r.x1 - r.x0) + (static_cast<uint32_t>(r.x0) + kPadX) % 4u) / kHospitalItem + 1u;
+}
+
+// Launch-table entry: (simulation, first item of its hospital scan).
 struct BlockRef {
   uint32_t sim, first;
 };

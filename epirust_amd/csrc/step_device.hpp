@@ -170,6 +170,10 @@ __device__ __forceinline__ uint32_t pack8(uint32_t top, uint32_t mid, uint32_t b
                              __builtin_amdgcn_udot4(bottom & kBit0, 0x00804020u, 0u, false), false),
       false);
 }
+// Four grid bytes (0..3) as four bits, set where occupied.
+__device__ __forceinline__ uint32_t occupied4(uint32_t bytes) {
+  return __builtin_amdgcn_udot4((bytes | (bytes >> 1)) & 0x01010101u, 0x08040201u, 0u, false);
+}
 // The vacant ones among the eight neighbours of the cell in byte 2 of the middle row; a
 // grid byte is 0..3, so a cell is occupied iff one of its two low bits is set.
 __device__ __forceinline__ uint32_t vacant8(uint64_t above, uint64_t row, uint64_t below) {
