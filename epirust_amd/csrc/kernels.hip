@@ -119,12 +119,13 @@ struct Agent {
   const SimDesc& D;
   const SimState& S;
   const uint8_t* __restrict__ occ;  // this simulation's grid
+  const uint32_t seed_lo, seed_hi;  // read up front too
   // Transmission thresholds, read once up front: a per-lane choice between two descriptor
   // fields would otherwise become a per-lane load of the chosen field.
   const uint64_t thr_regular, thr_high;
   uint32_t id, h, w, tm, wsa;
   uint32_t tm0 = 0;  // tm as stored: loaded for the states that carry an at_hour, else 0
-  const uint32_t* tm_arr = nullptr;  // this agent's stored tm word
+  uint32_t* tm_arr = nullptr;  // this agent's stored tm word
   int32_t x, y;                     // current cell
   int32_t tx, ty;                   // chosen cell
   int32_t hx = 0, hy = 0;           // home house origin (house id % H)
@@ -139,13 +140,13 @@ struct Agent {
   uint64_t r0 = 0, r1 = 0, r2 = 0, r3 = 0, r4 = 0;  // named, so no variable-index access exists
 
   __device__ Agent(const SimDesc& d, const SimState& s, const uint8_t* o)
-      : D(d), S(s), occ(o), thr_regular(Disease::transmission_threshold(d.dz, 1u)),
+      : D(d), S(s), occ(o), seed_lo(d.seed_lo), seed_hi(d.seed_hi), thr_regular(Disease::transmission_threshold(d.dz, 1u)),
         thr_high(Disease::transmission_threshold(d.dz, 2u)) {}
 
   __device__ __forceinline__ u32x4 dr(uint32_t site, uint32_t block) const {
-    return philox4x32_10(id, h, site, block, D.seed_lo, D.seed_hi);
+    return philox4x32_10(id, h, site, block, seed_lo, seed_hi);
   }
-  __device__ __forceinline__ void draw_move() { mv = philox4x32_9(id, h, SITE_MOVE, D.seed_lo, D.seed_hi); }
+  __device__ __forceinline__ void draw_move() { mv = philox4x32_9(id, h, SITE_MOVE, seed_lo, seed_hi); }
   __device__ __forceinline__ const u32x4& disease_words() const { return dz; }
 
   __device__ __forceinline__ uint32_t state() const { return fld(w, B_STATE, M_STATE); }
@@ -286,16 +287,15 @@ struct Agent {
 
   // default_disease_handler.rs:64-86 as an OR over fixed per-neighbour draws: first the
   // mask of eligible infectious neighbours of (tx, ty) from the window (rows chosen with
-  // bit masks, so no variable indexing), then one Philox block per pair of neighbours,
-  // drawn in Moore order only for eligible ones.
-  __device__ __forceinline__ bool on_susceptible() {
-    if (!Disease::can_catch(w)) return false;
-    const Rect a = current_area();
+  // bit masks, so no variable indexing), then the draws (infected_by).
+  uint32_t hot = 0, high = 0;  // infectious neighbours, in Moore order, and those in the high window
+  __device__ __forceinline__ void find_infectious() {
+    if (!Disease::can_catch(w)) return;
     cover(tx, ty);
     // No infectious cell (byte >= 2) anywhere in the 5 x 5 window, a superset of the
     // neighbourhood: nothing to test, and no draw is made. Most agents, and whole waves,
     // take this exit while infections are rare.
-    if (((r0 | r1 | r2 | r3 | r4) & 0xFEFEFEFEFEull) == 0) return false;
+    if (((r0 | r1 | r2 | r3 | r4) & 0xFEFEFEFEFEull) == 0) return;
     const int32_t ox = tx - wx, oy = ty - wy;  // both in [-1, 1]
     const uint64_t mm = oy < 0 ? ~0ull : 0ull, m0 = oy == 0 ? ~0ull : 0ull, mp = oy > 0 ? ~0ull : 0ull;
     const uint64_t top = (r0 & mm) | (r1 & m0) | (r2 & mp);
@@ -305,21 +305,26 @@ struct Agent {
     // high-window ones (byte 3) among the cells of the area and the grid
     const uint32_t c = static_cast<uint32_t>(ox + 1);
     const uint32_t bt = three(top, c), bm = three(mid, c), bb = three(bot, c);
-    const uint32_t ok = allowed8(a, tx, ty);
-    uint32_t hot = pack8(bt >> 1, bm >> 1, bb >> 1) & ok;
-    const uint32_t high = pack8(bt & (bt >> 1), bm & (bm >> 1), bb & (bb >> 1)) & ok;
+    const uint32_t infectious = pack8(bt >> 1, bm >> 1, bb >> 1);
+    if (infectious == 0) return;  // before the area's masks, which few agents need
+    hot = infectious & allowed8(current_area(), tx, ty);
+    high = pack8(bt & (bt >> 1), bm & (bm >> 1), bb & (bb >> 1)) & hot;
+  }
+  // The draws of agent `who` against its infectious neighbours: one Philox block per pair of
+  // neighbours, drawn in Moore order only for infectious ones.
+  __device__ __forceinline__ bool infected_by(uint32_t who, uint32_t infectious, uint32_t in_high) const {
     int blk = -1;
     uint32_t q0 = 0, q1 = 0, q2 = 0, q3 = 0;
-    while (hot) {
-      const int k = __builtin_ctz(hot);
-      hot &= hot - 1;
+    while (infectious) {
+      const int k = __builtin_ctz(infectious);
+      infectious &= infectious - 1;
       if ((k >> 1) != blk) {
         blk = k >> 1;
-        const u32x4 q = dr(SITE_INFECT, static_cast<uint32_t>(blk));
+        const u32x4 q = philox4x32_10(who, h, SITE_INFECT, static_cast<uint32_t>(blk), seed_lo, seed_hi);
         q0 = q.w[0]; q1 = q.w[1]; q2 = q.w[2]; q3 = q.w[3];
       }
       const uint64_t v = (k & 1) ? join64(q2, q3) : join64(q0, q1);
-      const uint64_t thr = ((high >> k) & 1u) ? thr_high : thr_regular;
+      const uint64_t thr = ((in_high >> k) & 1u) ? thr_high : thr_regular;
       if (bernoulli(thr, v)) return true;
     }
     return false;
@@ -331,11 +336,12 @@ struct Agent {
   }
 
   // DiseaseStateMachine::next (disease_state_machine.rs:53-70): the handler's transition of
-  // the current state; on_susceptible is the neighbour scan above.
+  // the current state; on_susceptible is the neighbour scan and the draws above.
   __device__ __forceinline__ void update_infection_dynamics() {
     const uint32_t s = state();
     if (s == ST_S) {
-      if (on_susceptible()) Disease::on_caught(h, w, tm);
+      find_infectious();
+      if (hot && infected_by(id, hot, high)) Disease::on_caught(h, w, tm);
     } else if (s == ST_E) {
       load_tm();
       Disease::on_exposed(D.dz, h, disease_words(), w, tm);
@@ -670,6 +676,8 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(const AgentBlock* bl
   bool whole_office = false;  // the claimed cell's office has all its slots in this block
   bool house_move = false;    // a home-layout move into the agent's own house
   uint64_t ci = 0;
+  uint32_t wsa0 = 0;
+  const uint32_t lane = threadIdx.x & (kWave - 1);
   // Office hours: the offices of this block's workers (j_lo .. j_hi, none in a block of
   // other agents and in the home layout), each with 100 cells in the block's claim filter.
   const uint32_t j_lo = first_lane(bm.j_lo), j_hi = first_lane(bm.j_hi);
@@ -692,12 +700,10 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(const AgentBlock* bl
     a.tx = a.x;
     a.ty = a.y;
     a.tm = 0;
-    const uint64_t gid = D.agent_off + local;  // tm and wsa stay in the home layout (by id)
+    const uint64_t gid = (ONE ? 0ull : bm.agent_off) + local;  // tm and wsa stay in the home layout (by id)
     a.tm_arr = v.tm + gid;
-    const uint32_t w0 = w_stored;
-    const bool staff = a.ws() == WS_STAFF;
-    a.wsa = staff ? v.wsa[gid] : 0u;
-    const uint32_t wsa0 = a.wsa;
+    a.wsa = wsa0 = a.ws() == WS_STAFF ? v.wsa[gid] : 0u;
+    w_in = w_stored;
 
     if (Disease::draws_needed(a.w, hd)) a.dz = a.dr(SITE_DISEASE, 0);
     if constexpr (C == HOURS_0) {
@@ -716,13 +722,7 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(const AgentBlock* bl
     key = claim_key(h, local);
     tgt_word = static_cast<uint32_t>(a.tx) | (static_cast<uint32_t>(a.ty) << 16);
     moves = tgt_word != p;
-    // the grid byte depends only on the state, the hospitalized flag, the infection day and
-    // the immunity, so it is recomputed only when one of those changed this hour
-    constexpr uint32_t kByteFields = (M_STATE << B_STATE) | F_HOSP | (M_DAY << B_DAY) | (M_IMM << B_IMM);
-    if (((a.w ^ w0) & kByteFields) && occupant_byte(D.dz, a.w) != occupant_byte(D.dz, w0)) a.w |= F_DIRTY;
     ci = D.cell_off + cell_index(D, a.tx, a.ty);
-    w_out = a.w;
-    w_in = w0;
     // a worker's claim of a cell of its own office (the only agents that claim office
     // cells at these hours) enters the filter
     const uint32_t j = fast_mod(local, D.fd_offices);  // the agent's office
@@ -740,8 +740,6 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(const AgentBlock* bl
     // the lowest-id claimant of such a cell is found among the agent's lower housemates,
     // whose target words the commit reads: no global claim is made.
     house_move = !office && moves && a.in_house(a.tx, a.ty);
-    if (a.tm != a.tm0) v.tm[gid] = a.tm;
-    if (staff && a.wsa != wsa0) v.wsa[gid] = a.wsa;
   }
   // Block claim filter (office hours). The office layout puts each office's workers in one
   // or two blocks, and they are the only claimants of its cells, so most same-cell rivals
@@ -760,6 +758,16 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(const AgentBlock* bl
     if (office_cell != kNoCell && s_cell[office_cell] != key) moves = false;
   }
   if (valid) {
+    // the grid byte depends only on the state, the hospitalized flag, the infection day and
+    // the immunity, so it is recomputed only when one of those changed this hour
+    constexpr uint32_t kByteFields = (M_STATE << B_STATE) | F_HOSP | (M_DAY << B_DAY) | (M_IMM << B_IMM);
+    if ((a.w ^ w_in) & kByteFields) {
+      const DiseaseParams dz = scalar_copy(&D.dz);
+      if (occupant_byte(dz, a.w) != occupant_byte(dz, w_in)) a.w |= F_DIRTY;
+    }
+    w_out = a.w;
+    if (a.tm != a.tm0) *a.tm_arr = a.tm;
+    if (a.wsa != wsa0) v.wsa[(ONE ? 0ull : bm.agent_off) + local] = a.wsa;
     if (moves) {
       if (whole_office) tgt_word |= kTgtWon;
       else if (house_move) tgt_word |= kTgtHouse;
@@ -774,7 +782,6 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(const AgentBlock* bl
   // the blocks'. Lanes without an agent hold no state.
   static_assert(ST_S == 0 && ST_E == 1 && ST_I == 2 && ST_R == 3 && ST_D == 4 && kNoState == 5 && B_STATE == 0, "bits");
   __shared__ uint32_t s_counts[kMaxWaves][8];
-  const uint32_t lane = threadIdx.x & (kWave - 1);
   const uint64_t b0 = __ballot(w_out & 1u), b1 = __ballot(w_out & 2u), b2 = __ballot(w_out & 4u);
   const uint64_t in_hospital = __ballot(w_out & F_HOSP), infected = b1 & ~b0;
   uint32_t mine = wave_count(~(b0 | b1 | b2));
