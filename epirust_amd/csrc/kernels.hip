@@ -642,11 +642,14 @@ __device__ __forceinline__ void epilogue_block(const DevView& v, const SimDesc* 
 // (kernel argument preload). ONE: the view has one simulation, whose descriptor and state need
 // not wait for the block's entry to name it. With both, an hour of 10k agents takes 7.08 -> 6.99
 // us, of 100k 7.99 -> 7.90, of 10M 150.9 -> 149.7 (with the preload alone 7.06, 8.00, 150.3).
-template <HourClass C, bool ONE>
+// HOME: hours of day 8..15 on the home layout, for days on which most agents are isolated and
+// stay at home or wherever the lockdown met them: nothing keeps a house's or an office's
+// claims to their own agents there then, so every move claims its cell.
+template <HourClass C, bool ONE, bool HOME>
 __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(const AgentBlock* blocks, const SimDesc* desc,
                                                             SimState* state, const uint32_t* st, const uint32_t* pos,
                                                             const uint32_t* ids, DevView v) {
-  constexpr bool office = on_office_layout(C);
+  constexpr bool office = on_office_layout(C) && !HOME;
   const AgentBlock bm = scalar_copy(blocks + blockIdx.x);
   const uint32_t count = first_lane(bm.count);
   // Every slot below the block's count holds an agent (the office slot map is a
@@ -689,7 +692,7 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(const AgentBlock* bl
   Agent a(D, *S, occ);
   a.id = local;
   a.h = h;
-  a.locate_buildings(office || C == HOURS_16);
+  a.locate_buildings(on_office_layout(C) || C == HOURS_16);
   if (C != HOURS_0 && C != HOURS_23) a.draw_move();
   loaded_together(w_stored, p, a.mv, active);
   if (!active) return;  // uniform over the block
@@ -732,14 +735,14 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(const AgentBlock* bl
                     static_cast<uint32_t>(a.tx - a.ox);
       whole_office = bm.whole != 0u;
     }
-    // Home-layout hours (16..23, 0..7): only a house's own agents (ids congruent mod
+    // Hours of day 16..23 and 0..7: only a house's own agents (ids congruent mod
     // n_houses) choose cells of that house. Local moves stay in the current area, which is
     // home for everyone but public-transport users (transport area) and hospital staff;
     // the teleports into a house (going home at 16, recovered going home at 23, the
     // hospital fallback at 0) are its own agents'; no one has the housing area then. So
     // the lowest-id claimant of such a cell is found among the agent's lower housemates,
     // whose target words the commit reads: no global claim is made.
-    house_move = !office && moves && a.in_house(a.tx, a.ty);
+    house_move = !on_office_layout(C) && moves && a.in_house(a.tx, a.ty);
   }
   // Block claim filter (office hours). The office layout puts each office's workers in one
   // or two blocks, and they are the only claimants of its cells, so most same-cell rivals
@@ -1139,28 +1142,31 @@ hipError_t launch_hospital_scan(const DevView& v, const LaunchShape& s, hipStrea
   return hipGetLastError();
 }
 
-template <HourClass C>
+template <HourClass C, bool HOME = false>
 hipError_t launch_step_class(const DevView& v, const LaunchShape& s, uint32_t blocks, uint32_t threads,
                              hipStream_t stream) {
-  const auto kernel = s.n_sims == 1 ? k_step<C, true> : k_step<C, false>;
+  const auto kernel = s.n_sims == 1 ? k_step<C, true, HOME> : k_step<C, false, HOME>;
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, stream, v.agent_blocks, v.desc, v.state, v.st, v.pos,
                      v.office_agent, v);
   return hipGetLastError();
 }
 
 hipError_t launch_step(const DevView& v, const LaunchShape& s, uint32_t hour, hipStream_t stream) {
-  const uint32_t blocks = v.office ? s.office_agent_blocks : s.agent_blocks;
+  const uint32_t hd = hour % 24u, blocks = v.office ? s.office_agent_blocks : s.agent_blocks;
   const uint32_t threads = v.office ? s.office_block : s.block;
   if (blocks == 0) return hipSuccess;
-  switch (hour % 24u) {
+  switch (hd) {
     case 0: return launch_step_class<HOURS_0>(v, s, blocks, threads, stream);
     case 7: case 17: return launch_step_class<HOURS_7_17>(v, s, blocks, threads, stream);
-    case 8: return launch_step_class<HOURS_8>(v, s, blocks, threads, stream);
+    case 8:
+      return v.office ? launch_step_class<HOURS_8>(v, s, blocks, threads, stream)
+                      : launch_step_class<HOURS_8, true>(v, s, blocks, threads, stream);
     case 16: return launch_step_class<HOURS_16>(v, s, blocks, threads, stream);
     case 23: return launch_step_class<HOURS_23>(v, s, blocks, threads, stream);
     default:
+      if (hd > 16u) return launch_step_class<HOURS_18_22>(v, s, blocks, threads, stream);
       return v.office ? launch_step_class<HOURS_9_15>(v, s, blocks, threads, stream)
-                      : launch_step_class<HOURS_18_22>(v, s, blocks, threads, stream);
+                      : launch_step_class<HOURS_9_15, true>(v, s, blocks, threads, stream);
   }
 }
 

@@ -68,10 +68,6 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
 
 // Lanes set in a wave's mask, and `x` with lane `lane` replaced, both on the scalar unit.
 __device__ __forceinline__ uint32_t wave_count(uint64_t mask) { return static_cast<uint32_t>(__builtin_popcountll(mask)); }
-__device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {  // of the mask's, below this one
-  return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32),
-                                   __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
-}
 template <int LANE>
 __device__ __forceinline__ uint32_t lane_word(uint32_t x, uint32_t value) {
   asm("v_writelane_b32 %0, %1, %2" : "+v"(x) : "s"(value), "n"(LANE));
