@@ -50,3 +50,34 @@ def test_runs_without_a_lockdown_in_such_a_batch(cfg1):
         assert batch.events(i) == cpu.events()
         cpu.close()
     batch.close()
+
+
+@pytest.mark.parametrize("hours", [5, 7, 8, 11, 15, 16, 24])
+def test_small_handle_moves_to_the_office_layout_when_its_blocks_are_set(cfg1, hours):
+    say("[home days] block size set after %d hours" % (24 + hours))
+    cfg = interventions_config(cfg1, n=3500, g=150)
+    gpu, cpu = G.Simulation(cfg), O.OracleSim(cfg)
+    for k in (24 + hours, 2, 70):
+        g_rows, _ = gpu.step(k)
+        c_rows, _ = cpu.step(k)
+        assert np.array_equal(g_rows, c_rows)
+        gpu.set_office_block_size(128)
+        assert_agents_equal(gpu.agents(), cpu.agents(), "a call of %d hours" % k)
+    gpu.close()
+    cpu.close()
+
+
+@pytest.mark.parametrize("n", [1, 64, 30000, 30001])
+def test_both_sides_of_the_size_that_has_an_office_layout(cfg1, n):
+    say("[home days] %d agents" % n)
+    cfg = config(cfg1, n, max(60, int(2.2 * n ** 0.5)), 0, 0)
+    cfg["starting_infections"] = {"exposed": min(n, 30), "infected_mild_asymptomatic": 0,
+                                  "infected_mild_symptomatic": 0, "infected_severe": 0}
+    gpu, cpu = G.Simulation(cfg), O.OracleSim(cfg)
+    for k in (13, 30):
+        g_rows, _ = gpu.step(k)
+        c_rows, _ = cpu.step(k)
+        assert np.array_equal(g_rows, c_rows)
+        assert_agents_equal(gpu.agents(), cpu.agents(), "a call of %d hours" % k)
+    gpu.close()
+    cpu.close()
