@@ -120,7 +120,7 @@ struct epi_sim {
   std::vector<SimDesc> desc;
   std::vector<uint32_t> counts0;  // 7 per sim
   uint32_t n_sims = 0;
-  uint64_t n_agents = 0, n_cells = 0, n_rows = 0, n_events = 0;
+  uint64_t n_agents = 0, n_cells = 0, n_grid = 0, n_rows = 0, n_events = 0;
   uint32_t max_hour = 0;  // largest hour any simulation can reach
   bool any_empty = false;
   uint32_t flags = 0;
@@ -743,7 +743,7 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
   s->counts0.resize(7 * s->n_sims);
   s->rows_returned.assign(s->n_sims, 0);
   s->state_h.resize(s->n_sims);
-  uint64_t agent_off = 0, cell_off = 0, row_off = 0, event_off = 0;
+  uint64_t agent_off = 0, cell_off = 0, grid_off = 0, row_off = 0, event_off = 0;
   for (uint32_t i = 0; i < s->n_sims; ++i) {
     const Config& c = s->cfg[i];
     const Geometry& G = pops[i].geo;
@@ -754,10 +754,12 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
     D.g = G.g;
     D.stride = G.stride;
     D.pitch = padded_pitch(G.stride);
+    D.strip = strip_bytes(G.height);
     D.height = G.height;
     D.hours = c.hours;
     D.agent_off = agent_off;
     D.cell_off = cell_off;
+    D.grid_off = grid_off;
     D.row_off = row_off;
     D.event_off = event_off;
     D.event_cap = 4u + static_cast<uint32_t>(c.vaccinate.size()) + 2u * (c.hours / 24u + 1u);
@@ -805,6 +807,7 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
     if (c.number_of_agents == 0 && c.hours > 1) s->any_empty = true;
     agent_off += D.n_slots;
     cell_off += padded_cells(G.stride, G.height);
+    grid_off += grid_bytes(G.stride, G.height);
     row_off += c.hours > 1 ? c.hours - 1 : 0;
     event_off += D.event_cap;
     s->max_hour = std::max(s->max_hour, c.hours > 1 ? c.hours - 1 : 0u);
@@ -817,6 +820,7 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
   }
   s->n_agents = agent_off;
   s->n_cells = cell_off;
+  s->n_grid = grid_off;
   s->n_rows = row_off;
   s->n_events = event_off;
   s->shape.hosp_blocks = static_cast<uint32_t>(s->hosp_blocks.size());
@@ -841,7 +845,7 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
   DevView& vo = s->v_office;  // completed from v below
   HIP_TRY(M.alloc(&vo.pos, s->n_agents));
   HIP_TRY(M.alloc(&vo.st, s->n_agents));
-  HIP_TRY(M.alloc(&v.occ, s->n_cells));
+  HIP_TRY(M.alloc(&v.occ, s->n_grid));
   HIP_TRY(M.alloc(&v.claim, s->n_cells));
   HIP_TRY(M.alloc(&s->d_desc, s->n_sims));
   v.desc = s->d_desc;
@@ -889,7 +893,7 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
     s->state_h[i] = st;
     if (!host_init) {
       jobs.push_back(InitJob{&s->cfg[i], s->seed[i], &P.geo, v.pos + D.agent_off, v.st + D.agent_off,
-                             v.tm + D.agent_off, v.wsa + D.agent_off, v.occ + D.cell_off, D.pitch});
+                             v.tm + D.agent_off, v.wsa + D.agent_off, v.occ + D.grid_off, D.strip});
       continue;
     }
     if (D.n) {
@@ -898,17 +902,16 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
       HIP_TRY(hipMemcpy(v.tm + D.agent_off, P.tm.data(), nb, hipMemcpyHostToDevice));
       HIP_TRY(hipMemcpy(v.wsa + D.agent_off, P.wsa.data(), nb, hipMemcpyHostToDevice));
     }
-    const size_t cells = padded_cells(P.geo.stride, P.geo.height);
-    grid.assign(cells, 0);
+    grid.assign(grid_bytes(P.geo.stride, P.geo.height), 0);
     for (uint32_t a = 0; a < D.n; ++a) {
-      const uint32_t p = P.pos[a];
-      grid[static_cast<size_t>((p >> 16) + kPadY) * D.pitch + (p & 0xFFFFu) + kPadX] =
-          occupant_byte(D.dz, P.st[a]);
+      const GridPlace g = grid_place(D.strip, P.pos[a] & 0xFFFFu, P.pos[a] >> 16);
+      grid[g.at] = occupant_byte(D.dz, P.st[a]);
+      if (in_two_strips(g)) grid[second_place(D.strip, g)] = grid[g.at];
     }
-    HIP_TRY(hipMemcpy(v.occ + D.cell_off, grid.data(), cells, hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(v.occ + D.grid_off, grid.data(), grid.size(), hipMemcpyHostToDevice));
   }
   if (!jobs.empty()) {
-    HIP_TRY(hipMemsetAsync(v.occ, 0, s->n_cells, s->stream));
+    HIP_TRY(hipMemsetAsync(v.occ, 0, s->n_grid, s->stream));
     std::string err;
     const hipError_t e = synthesize_on_device(jobs, s->stream, err);
     if (e != hipSuccess) return fail(EPI_ERR_DEVICE, "device population synthesis (" + err + "): " + hipGetErrorString(e));

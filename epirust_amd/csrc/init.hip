@@ -18,7 +18,7 @@
 //                    rank test against the scanned counts, then its group of starting
 //                    infections from the four rank bounds;
 //   k_init_cells   : per house, random_points(k) of the 2x2 house for its agents, and their
-//                    bytes of the padded occupancy grid.
+//                    bytes of the occupancy grid.
 // All of it is integer work over a few bytes per agent and runs once per handle, a chain of
 // launches that nothing on the host waits for: 32 simulations of 100k agents are created in
 // 13.1 -> 1.7 ms, 64 of mixed sizes in 26.8 -> 3.3, one of 10k in 0.57 -> 0.46 (before: a simulation at a
@@ -63,7 +63,7 @@ struct InitSim {
   uint32_t* tm;
   uint32_t* wsa;
   uint8_t* occ;
-  uint32_t pitch;
+  uint32_t strip;
   DiseaseParams dz;
   int32_t house_sx, house_sy, house_nx;
   uint32_t n_houses;
@@ -382,7 +382,10 @@ __global__ __launch_bounds__(kInitBlock) void k_init_cells(const InitSim* sims, 
     for (uint32_t q = 0; q < my && j < k; ++q, ++j) {
       const uint32_t id = h + j * H, x = static_cast<uint32_t>(xs[p]), y = static_cast<uint32_t>(ys[q]);
       a.pos[id] = x | (y << 16);
-      a.occ[static_cast<size_t>(y + kPadY) * a.pitch + x + kPadX] = occupant_byte(a.dz, a.st[id]);
+      const uint8_t byte = occupant_byte(a.dz, a.st[id]);
+      const GridPlace g = grid_place(a.strip, x, y);
+      a.occ[g.at] = byte;
+      if (in_two_strips(g)) a.occ[second_place(a.strip, g)] = byte;
     }
 }
 
@@ -533,7 +536,7 @@ hipError_t synthesize_on_device(const std::vector<InitJob>& jobs, hipStream_t st
     a.tm = jobs[i].tm;
     a.wsa = jobs[i].wsa;
     a.occ = jobs[i].occ;
-    a.pitch = jobs[i].pitch;
+    a.strip = jobs[i].strip;
     a.dz = Disease::params(cfg);
     a.house_sx = geo.house_sx;
     a.house_sy = geo.house_sy;

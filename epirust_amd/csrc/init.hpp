@@ -14,14 +14,14 @@
 namespace epi {
 
 // One simulation: what to build, and its slices of the batch's concatenated arrays. The grid
-// (padded, `pitch`) must be clear.
+// (strips of `strip` bytes) must be clear.
 struct InitJob {
   const Config* cfg;
   uint64_t seed;
   const Geometry* geo;
   uint32_t *pos, *st, *tm, *wsa;
   uint8_t* occ;
-  uint32_t pitch;
+  uint32_t strip;
 };
 
 // Fills the jobs' slices with the same agents synthesize_population builds on the host, on

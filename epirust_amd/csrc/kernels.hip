@@ -197,7 +197,7 @@ struct Agent {
   __device__ __forceinline__ void set_area(uint32_t tag) { w = set_fld(w, B_AREA, M_AREA, tag); }
 
   __device__ __forceinline__ bool vacant(int32_t cx, int32_t cy) const {
-    return occ[cell_index(D, cx, cy)] == 0;
+    return occ[grid_place(D.strip, static_cast<uint32_t>(cx), static_cast<uint32_t>(cy)).at] == 0;
   }
   // The cells around (cx, cy) that lie in rect a and in the grid (area.rs:83-88 and
   // allocation_map.rs:156-159 for each neighbour), in the order of the eight neighbours.
@@ -213,18 +213,20 @@ struct Agent {
   }
   // Five independent loads of the two aligned words that hold columns cx-2..cx+2 of a row (an
   // unaligned eight-byte load takes twice the L1 accesses: 10M agents 161 us an hour, 153 with
-  // these), from one offset on five uniform row bases, then shifted to column cx-2.
+  // these), a strip's row apart, then shifted to column cx-2.
   __device__ __forceinline__ void load_window(int32_t cx, int32_t cy) {
-    const uint32_t px = static_cast<uint32_t>(cx) + (kPadX - 2u);
-    const uint32_t off = __umul24(static_cast<uint32_t>(cy) + (kPadY - 2u), D.pitch) + (px & ~3u);
+    const uint32_t first = static_cast<uint32_t>(cx) + (kPadX - 2u), k = strip_of(first);
+    const uint32_t b = first - k * kStripStep;
+    const uint32_t off = strip_start(D.strip, k) + (static_cast<uint32_t>(cy) + (kPadY - 2u)) * kStripRow + (b & ~3u);
+    const GlobalBytes base = (GlobalBytes)occ;
     uint2 q[5];
 #pragma unroll
-    for (uint32_t r = 0; r < 5; ++r) q[r] = load_words2(uniform_base(occ + r * D.pitch), off);
-    r0 = from_byte(q[0], px & 3u);
-    r1 = from_byte(q[1], px & 3u);
-    r2 = from_byte(q[2], px & 3u);
-    r3 = from_byte(q[3], px & 3u);
-    r4 = from_byte(q[4], px & 3u);
+    for (uint32_t r = 0; r < 5; ++r) q[r] = load_words2(base + r * kStripRow, off);
+    r0 = from_byte(q[0], b & 3u);
+    r1 = from_byte(q[1], b & 3u);
+    r2 = from_byte(q[2], b & 3u);
+    r3 = from_byte(q[3], b & 3u);
+    r4 = from_byte(q[4], b & 3u);
     wx = cx;
     wy = cy;
   }
@@ -671,7 +673,7 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(const AgentBlock* bl
   constexpr uint32_t kFirst = first_hour(C), kLast = last_hour(C);
   __builtin_assume(hd >= kFirst && hd <= kLast);
   const Sweep sweep = sweep_slot(*S, (h - 1u) & 1u);  // decided at hour h - 1
-  const uint8_t* occ = v.occ + D.cell_off;
+  const uint8_t* occ = v.occ + D.grid_off;
 
   // This lane's claim and state word, carried past the block's claim filter to the stores.
   bool moves = false;
@@ -878,6 +880,13 @@ __device__ __forceinline__ void rest_pass(const DevView& v, const SimDesc& D, co
   reset_claims(share);
 }
 
+// The grid byte of cell `c` (x | y << 16), in both its places.
+__device__ __forceinline__ void put_byte(uint8_t* occ, uint32_t strip, uint32_t c, uint8_t byte) {
+  const GridPlace g = grid_place(strip, c & 0xFFFFu, c >> 16);
+  occ[g.at] = byte;
+  if (in_two_strips(g)) occ[second_place(strip, g)] = byte;
+}
+
 // `parity` is the hour's parity (an hour of day 24k + j has the parity of j). Blocks
 // 0 .. n_epi-1 run the epilogue of simulation blockIdx.x; the rest run the agent pass:
 // the commit at hours of day 0 and 7..23, rest_pass at 1..6. Eight waves per SIMD (64 VGPRs)
@@ -932,8 +941,8 @@ __global__ __attribute__((amdgpu_waves_per_eu(8))) void k_commit(const AgentBloc
       const uint64_t cell_off = scalar_copy(&D.cell_off);
       const uint32_t pitch = scalar_copy(&D.pitch);
       const DiseaseParams dz = scalar_copy(&D.dz);
-      uint8_t* occ = v.occ + cell_off;
-      const uint32_t old_ci = cell_index(pitch, static_cast<int32_t>(p & 0xFFFFu), static_cast<int32_t>(p >> 16));
+      const uint32_t strip = scalar_copy(&D.strip);
+      uint8_t* occ = v.occ + scalar_copy(&D.grid_off);
       const uint8_t byte = occupant_byte(dz, w);
       bool moved = false;
       if (mover) {
@@ -945,13 +954,13 @@ __global__ __attribute__((amdgpu_waves_per_eu(8))) void k_commit(const AgentBloc
         t &= kTgtCell;
         const uint32_t ci = cell_index(pitch, static_cast<int32_t>(t & 0xFFFFu), static_cast<int32_t>(t >> 16));
         if (won || (!house && (v.claim + cell_off)[ci] == claim_key(h, local))) {
-          occ[old_ci] = 0;
-          occ[ci] = byte;
+          put_byte(occ, strip, p, 0);
+          put_byte(occ, strip, t, byte);
           pos[gi] = t;
           moved = true;
         }
       }
-      if (!moved && (w & F_DIRTY)) occ[old_ci] = byte;
+      if (!moved && (w & F_DIRTY)) put_byte(occ, strip, p, byte);
       if (w & F_DIRTY) st[gi] = w & ~F_DIRTY;
     }
   }
@@ -974,11 +983,11 @@ __global__ void k_apply_sweep(DevView v) {
 }
 
 // First vacant cell of the current hospital area in row-major order (area.rs:119-146 +
-// allocation_map.rs:145) of the snapshot grid. A thread takes 16 cells of a row at a time, the
+// allocation_map.rs:145) of the snapshot grid. A thread takes a strip's 60 cells of a row, the
 // items of a block in row-major order too, so the block's first vacant cell is the one of its
 // first wave and lane that has any. One atomicMin per block that beats what is there: atomics to
 // one address, from every wave of a mostly vacant hospital, were the scan's time (10M agents
-// 109 -> 15 us a day).
+// 109 -> 15 us a day; 7 with a strip's row per thread).
 __global__ void k_hospital_scan(DevView v, uint32_t items_per_thread) {
   __shared__ uint32_t s_first[kMaxWaves];
   const BlockRef bm = v.hosp_blocks[blockIdx.x];
@@ -990,12 +999,13 @@ __global__ void k_hospital_scan(DevView v, uint32_t items_per_thread) {
   const uint32_t wd = static_cast<uint32_t>(hr.x1 - hr.x0 + 1), rows = static_cast<uint32_t>(hr.y1 - hr.y0 + 1);
   const uint32_t per_row = hospital_items(hr), n = per_row * rows;
   if (first >= n) return;
-  const uint32_t lead = (static_cast<uint32_t>(hr.x0) + kPadX) & 3u;  // bytes of a row's first item before the area
+  const uint32_t strip0 = strip_of(static_cast<uint32_t>(hr.x0) + kPadX);
+  const uint32_t lead = static_cast<uint32_t>(hr.x0) + kPadX - strip0 * kStripStep;  // of the first item, before the area
   const uint32_t row0 = first / per_row, item0 = first - row0 * per_row;
-  const uint32_t cell0 = row0 * wd + (item0 ? item0 * kHospitalItem - lead : 0u);  // the block's first cell
+  const uint32_t cell0 = row0 * wd + (item0 ? item0 * kStripStep - lead : 0u);  // the block's first cell
   if (__hip_atomic_load(&S->first_vacant, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < cell0)
     return;  // an earlier block already found one
-  const uint8_t* occ = v.occ + D.cell_off;
+  const uint8_t* occ = v.occ + D.grid_off;
   const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, waves = blockDim.x / kWave;
   uint32_t best = ~0u;
   for (uint32_t k = 0; k < items_per_thread && best == ~0u; ++k) {  // uniform over the wave
@@ -1003,16 +1013,20 @@ __global__ void k_hospital_scan(DevView v, uint32_t items_per_thread) {
     const uint32_t row = q / per_row, item = q - row * per_row;
     uint32_t mine = ~0u;
     if (q < n) {
-      const uint32_t x = (static_cast<uint32_t>(hr.x0) + kPadX - lead) + item * kHospitalItem;
       const uint32_t y = static_cast<uint32_t>(hr.y0) + row + kPadY;
-      typedef uint4 Words __attribute__((aligned(4)));
-      const uint4 b = *reinterpret_cast<const Words*>(occ + (static_cast<size_t>(y) * D.pitch + x));
+      const uint4* words = reinterpret_cast<const uint4*>(occ + (static_cast<size_t>(strip0 + item) * D.strip + y * kStripRow));
       // a bit per vacant cell (grid bytes are 0..3), those outside the area left out
-      uint32_t vacant = ~(occupied4(b.x) | (occupied4(b.y) << 4) | (occupied4(b.z) << 8) | (occupied4(b.w) << 12)) & 0xFFFFu;
-      const uint32_t past = wd + lead - item * kHospitalItem;  // bytes of the area from this item on
-      if (item == 0) vacant &= ~0u << lead;
-      if (past < kHospitalItem) vacant &= (1u << past) - 1u;
-      if (vacant) mine = row * wd + item * kHospitalItem - lead + static_cast<uint32_t>(__builtin_ctz(vacant));
+      uint64_t occupied = 0;
+#pragma unroll
+      for (uint32_t c = 0; c < kStripRow / 16u; ++c) {
+        const uint4 b = words[c];
+        occupied |= static_cast<uint64_t>(occupied4(b.x) | (occupied4(b.y) << 4) | (occupied4(b.z) << 8) | (occupied4(b.w) << 12)) << (16u * c);
+      }
+      uint64_t vacant = ~occupied & ((1ull << kStripStep) - 1u);
+      const uint32_t past = wd + lead - item * kStripStep;  // cells of the area from this item's first on
+      if (item == 0) vacant &= ~0ull << lead;
+      if (past < kStripStep) vacant &= (1ull << past) - 1u;
+      if (vacant) mine = row * wd + item * kStripStep - lead + static_cast<uint32_t>(__builtin_ctzll(vacant));
     }
     const uint64_t found = __ballot(mine != ~0u);
     if (found) best = __shfl(mine, __builtin_ctzll(found), kWave);

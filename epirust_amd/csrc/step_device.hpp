@@ -96,7 +96,7 @@ __device__ __forceinline__ uint32_t set_fld(uint32_t w, uint32_t b, uint32_t m, 
   return (w & ~(m << b)) | ((v & m) << b);
 }
 
-// Index of cell (x, y) in the padded grid / claim arrays of one simulation. A simulation
+// Index of cell (x, y) in the claim array of one simulation. A simulation
 // has fewer than 2^32 padded cells (grid_size <= 32,000), so the index is 32-bit and a
 // load adds it to the simulation's base as an unsigned offset.
 __device__ __forceinline__ uint32_t cell_index(uint32_t pitch, int32_t x, int32_t y) {
@@ -137,15 +137,7 @@ __device__ __forceinline__ uint32_t span3(int32_t base, int32_t lo, int32_t hi) 
   return (0x7u << from) & (0x7u >> past) & 0x7u;
 }
 
-// A pointer that is the same in all lanes, kept in scalar registers: a load adds the lane's
-// 32-bit offset to it in the instruction, where the compiler would otherwise fold the pointer
-// into the lane's part and pay a 64-bit vector add per load.
 typedef const __attribute__((address_space(1))) uint8_t* GlobalBytes;
-__device__ __forceinline__ GlobalBytes uniform_base(const uint8_t* p) {
-  GlobalBytes q = (GlobalBytes)p;
-  asm("" : "+s"(q));
-  return q;
-}
 // Two words at base + off, off a multiple of 4.
 __device__ __forceinline__ uint2 load_words2(GlobalBytes base, uint32_t off) {
   typedef uint64_t Words __attribute__((aligned(4)));
