@@ -150,7 +150,8 @@ struct epi_sim {
   std::vector<uint8_t> day_flags;
   SimDesc* d_desc = nullptr;
   hipStream_t stream = nullptr;
-  hipGraphExec_t day_graph[DAY_VARIANTS] = {};  // by the day's flags
+  hipGraphExec_t day_graph[DAY_VARIANTS] = {};   // by the day's flags
+  hipGraphExec_t days_graph[DAY_VARIANTS] = {};  // kGraphDays of them
   hipEvent_t poll_event[2] = {nullptr, nullptr};
   hipEvent_t loop_event[2] = {nullptr, nullptr};  // around the hour loop of one step call
   double last_loop_ms = 0.0;                      // device time of the last step call's hours
@@ -174,6 +175,8 @@ struct epi_sim {
 
   ~epi_sim() {
     for (hipGraphExec_t g : day_graph)
+      if (g) (void)hipGraphExecDestroy(g);
+    for (hipGraphExec_t g : days_graph)
       if (g) (void)hipGraphExecDestroy(g);
     for (auto& e : poll_event)
       if (e) (void)hipEventDestroy(e);
@@ -436,7 +439,7 @@ int enqueue_hour(epi_sim* s, uint32_t next_hour, bool home_day = false) {
 }
 
 // Whether at least half of all agents are under a lockdown that isolates them, by the states that
-// the host has so far (a few days old while a call runs ahead). They stay where they are, so
+// the host has so far (up to two graphs old while a call runs ahead). They stay where they are, so
 // the office layout's neighbours are not neighbours then (10M agents with a lockdown on day 22 of
 // 60: 144.3 us an hour on the office layout throughout, 134.5 with this rule, 172 on the home
 // layout throughout; 32 runs of 100k with one: 43.9, 40.8, 51.4). Either gives the same results.
@@ -446,6 +449,20 @@ bool mostly_isolated(const epi_sim* s) {
     if (const_cast<const volatile SimState*>(s->pinned_state)[i].locked)
       isolated += static_cast<double>(s->desc[i].n) * (1.0 - s->cfg[i].essential_workers_population);
   return 2.0 * isolated >= static_cast<double>(s->n_agents) && s->n_agents != 0;
+}
+
+// Days of equal flags that one graph runs in handles of at most kGraphAgents: between two graphs
+// lie the active flags' export and its event, 6.5 us (an hour of 10k agents 6.50 us with a graph
+// per day, 6.22 with four days; 100k 7.40, 7.22; 1M 18.40, 18.12; 32 runs of 100k 40.35, 39.87).
+// Larger ones gain less than they lose to the later sight of a lockdown (mostly_isolated).
+constexpr uint32_t kGraphDays = 4;
+constexpr uint64_t kGraphAgents = 4000000;
+uint32_t graph_days(const epi_sim* s, uint32_t target) {
+  if (s->n_agents > kGraphAgents || target - s->host_hour < 24u * kGraphDays) return 1;
+  const uint8_t* flags = &s->day_flags[s->host_hour / 24u];
+  for (uint32_t d = 1; d < kGraphDays; ++d)
+    if (flags[d] != flags[0]) return 1;
+  return kGraphDays;
 }
 
 // The groups of hours that the day from `hour` + 1 on runs as one launch each.
@@ -482,21 +499,23 @@ int enqueue_hours_plain(epi_sim* s, uint32_t first, uint32_t last) {
   return EPI_OK;
 }
 
-int capture_day_graph(epi_sim* s, uint8_t flags) {
-  if (s->day_graph[flags]) return EPI_OK;
+int capture_days(epi_sim* s, uint8_t flags, uint32_t days, hipGraphExec_t& exec) {
+  if (exec) return EPI_OK;
   hipGraph_t graph = nullptr;
   HIP_TRY(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-  const int rc = enqueue_hours(s, 1, 24, flags);  // the hours of day of 24d+1 .. 24d+24
+  int rc = EPI_OK;
+  for (uint32_t d = 0; d < days && rc == EPI_OK; ++d)
+    rc = enqueue_hours(s, 1, 24, flags);  // the hours of day of 24d+1 .. 24d+24
   hipError_t e = hipStreamEndCapture(s->stream, &graph);
   if (rc != EPI_OK) {
     if (graph) (void)hipGraphDestroy(graph);
     return rc;
   }
   if (e != hipSuccess) return fail(EPI_ERR_DEVICE, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-  e = hipGraphInstantiate(&s->day_graph[flags], graph, nullptr, nullptr, 0);
+  e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
   (void)hipGraphDestroy(graph);
   if (e != hipSuccess) {
-    s->day_graph[flags] = nullptr;
+    exec = nullptr;
     return fail(EPI_ERR_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
   }
   return EPI_OK;
@@ -597,7 +616,7 @@ int advance(epi_sim* s, uint32_t target) {
   uint32_t day_index = 0;
   bool pending[2] = {false, false};
   while (s->host_hour < target) {
-    // poll the flags copied two days ago
+    // poll the flags copied two graphs ago
     const uint32_t slot = day_index & 1u;
     if (pending[slot]) {
       HIP_TRY(hipEventSynchronize(s->poll_event[slot]));
@@ -606,10 +625,12 @@ int advance(epi_sim* s, uint32_t target) {
     }
     if (graph_ok && s->host_hour % 24u == 0 && target - s->host_hour >= 24u) {
       const uint8_t flags = flags_of_day(s, s->host_hour) | (mostly_isolated(s) ? DAY_HOME : 0);
-      int rc = capture_day_graph(s, flags);
+      const uint32_t days = graph_days(s, target);
+      hipGraphExec_t& exec = days > 1 ? s->days_graph[flags] : s->day_graph[flags];
+      int rc = capture_days(s, flags, days, exec);
       if (rc != EPI_OK) return rc;
-      HIP_TRY(hipGraphLaunch(s->day_graph[flags], s->stream));
-      s->host_hour += 24;
+      HIP_TRY(hipGraphLaunch(exec, s->stream));
+      s->host_hour += 24u * days;
     } else {
       const uint32_t end = std::min(target, (s->host_hour / 24u + 1u) * 24u);
       const int rc = graph_ok ? enqueue_hours(s, s->host_hour + 1, end, flags_of_day(s, s->host_hour))
@@ -1435,11 +1456,12 @@ static int set_launch_blocks(epi_sim* sim, uint32_t home, uint32_t office) {
     rc = relayout(sim, true);
     if (rc != EPI_OK) return rc;
   }
-  for (hipGraphExec_t& g : sim->day_graph)
-    if (g) {
-      (void)hipGraphExecDestroy(g);
-      g = nullptr;
-    }
+  for (hipGraphExec_t* graphs : {sim->day_graph, sim->days_graph})
+    for (uint32_t f = 0; f < DAY_VARIANTS; ++f)
+      if (graphs[f]) {
+        (void)hipGraphExecDestroy(graphs[f]);
+        graphs[f] = nullptr;
+      }
   return EPI_OK;
 }
 

@@ -65,3 +65,20 @@ def test_counts_of_many_blocks(cfg1, n):
     assert np.array_equal(g_rows, c_rows)
     gpu.close()
     cpu.close()
+
+
+# Graphs of one and of four days, runs that end inside one, and days of other groups between them.
+@pytest.mark.parametrize("vaccinate", [(), (74,), (25, 221)])
+@pytest.mark.parametrize("calls", [(95,), (96,), (97, 240), (24, 400)])
+def test_calls_of_many_days(cfg1, vaccinate, calls):
+    say("[day groups] calls of %s hours, vaccinations at %s" % (calls, vaccinate))
+    cfg = small(cfg1, vaccinate, hours=420)
+    gpu, cpu = G.Simulation(cfg), O.OracleSim(cfg)
+    for k in calls:
+        g_rows, g_stop = gpu.step(k)
+        c_rows, c_stop = cpu.step(k)
+        assert np.array_equal(g_rows, c_rows) and g_stop == c_stop
+        assert_agents_equal(gpu.agents(), cpu.agents(), "a call of %d hours" % k)
+    assert gpu.events() == cpu.events()
+    gpu.close()
+    cpu.close()
