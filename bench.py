@@ -47,7 +47,8 @@ def tuned_shape_of(cfg, block=None):
     from epirust_amd import autotune
     if block:
         return block, block
-    default = 512 if cfg["population"]["Auto"]["number_of_agents"] >= (1 << 19) else 256
+    n = cfg["population"]["Auto"]["number_of_agents"]
+    default = 128 if n <= 30000 else 256 if n < (1 << 16) else 512
     return autotune.tuned_shape([cfg]) or (default, default)
 
 

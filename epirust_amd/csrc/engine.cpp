@@ -846,11 +846,14 @@ int create_impl(const std::vector<std::string>& texts, const std::vector<uint64_
   s->n_events = event_off;
   s->shape.hosp_blocks = static_cast<uint32_t>(s->hosp_blocks.size());
   s->shape.n_sims = s->n_sims;
-  // Default threads per agent block, as measured on MI355X: 512 for one simulation of at
-  // least 2^19 agents (1M agents: 31 against 33 µs per hour at 256; 10M: 231 against 250),
-  // 256 for batches and smaller runs, the same at office hours. epi_set_block_size
-  // overrides both, epi_set_office_block_size then the office layout's alone.
-  s->shape.block = (s->n_sims == 1 && s->desc[0].n >= (1u << 19)) ? 512u : 256u;
+  // Default threads per agent block, as measured on MI355X, for one simulation: 128 up to
+  // kHomeAgents, where a launch is as long as its last block (us an hour at 128, 256, 512: 2k agents
+  // 6.45, 6.65, 6.84; 10k 6.07, 6.32, 6.56; 25k 6.48, 6.61, 6.83), 512 from 2^16 agents on (256, 512:
+  // 40k 6.96, 7.05; 60k 7.07, 7.05; 100k 7.19, 6.98; 333k 11.56, 11.47; 1M 18.91, 18.53; 10M 140.9,
+  // 139.8), 256 between and for batches (32 x 100k 42.7, 43.6; 64 of mixed sizes 126.9, 129.8), the
+  // same at office hours. epi_set_block_size overrides both, epi_set_office_block_size then the
+  // office layout's alone.
+  s->shape.block = s->n_sims > 1 ? 256u : s->n_agents <= kHomeAgents ? 128u : s->n_agents < (1u << 16) ? 256u : 512u;
   s->shape.office_block = s->shape.block;
   set_day_flags(s.get());
 

@@ -166,9 +166,9 @@ int epi_last_run_ms(epi_sim* sim, double* device_ms, uint32_t* hours);
 
 /* Launch shape (no reference counterpart): threads per agent block (64..1024, multiple of
  * 64), for the home and the office layout alike. Takes effect on the next step; discards
- * the captured day graph. Default: 512 for a single simulation of at least 2^19 agents,
- * else 256. A handle of at most 30,000 agents runs office hours on the home layout until
- * this or the next function is called. */
+ * the captured day graphs. Default: 128 for a single simulation of at most 30,000 agents,
+ * 512 for one of at least 2^16, else 256. A handle of at most 30,000 agents runs office
+ * hours on the home layout until this or the next function is called. */
 int epi_set_block_size(epi_sim* sim, uint32_t threads);
 
 /* Launch shape (no reference counterpart): threads per agent block of the office layout

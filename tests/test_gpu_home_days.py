@@ -67,7 +67,7 @@ def test_small_handle_moves_to_the_office_layout_when_its_blocks_are_set(cfg1, h
     cpu.close()
 
 
-@pytest.mark.parametrize("n", [1, 64, 30000, 30001])
+@pytest.mark.parametrize("n", [1, 64, 30000, 30001, 65535, 65536])
 def test_both_sides_of_the_size_that_has_an_office_layout(cfg1, n):
     say("[home days] %d agents" % n)
     cfg = config(cfg1, n, max(60, int(2.2 * n ** 0.5)), 0, 0)
