@@ -336,7 +336,7 @@ int build_launch_tables(epi_sim* s) {
 
 // The office layout's slot order (model.hpp): per simulation, the Normal and Essential
 // workers office by office (office = id % n_offices), each office's in id order, then the
-// other agents in id order. Work statuses are fixed at creation, so the slot maps are
+// other agents house by house. Work statuses are fixed at creation, so the slot maps are
 // built once, on the device from the synthesized state words, with the layout move's tiles.
 // Most agents of a handle whose office hours need no office layout: its two moves a day cost more
 // launches than its neighbours save (an hour of 20k agents 7.13 us with it, 6.83 without; of 40k
@@ -347,7 +347,7 @@ int build_office_order(epi_sim* s) {
   std::vector<OfficeJob> jobs;
   for (uint32_t i = 0; i < s->n_sims; ++i) {
     const SimDesc& D = s->desc[i];
-    jobs.push_back(OfficeJob{D.n, D.n_offices, s->v.st + D.agent_off, s->d_office_agent + D.agent_off,
+    jobs.push_back(OfficeJob{D.n, D.n_offices, D.n_houses, s->v.st + D.agent_off, s->d_office_agent + D.agent_off,
                              s->d_office_slot + D.agent_off});
   }
   std::string err;

@@ -31,7 +31,7 @@ hipError_t synthesize_on_device(const std::vector<InitJob>& jobs, hipStream_t st
 
 // One simulation's office layout (model.hpp) from its home-layout state words `st` (n agents).
 struct OfficeJob {
-  uint32_t n, n_offices;
+  uint32_t n, n_offices, n_houses;
   const uint32_t* st;
   uint32_t *office_agent, *office_slot;
 };

@@ -25,7 +25,7 @@
 //   k_relayout: [hours of day 8 and 16] moves st and pos between the home layout
 //              (slot = agent id) and the office layout that hours of day 8..15 run on:
 //              each office's workers in consecutive slots, packed whole into blocks,
-//              then everyone else in id order. There k_step resolves the claims of each
+//              then everyone else house by house. There k_step resolves the claims of each
 //              office's cells among the block's workers in LDS, and the winners on
 //              offices that lie wholly in one block (all of them when an office fits a
 //              block) claim nothing globally.

@@ -155,7 +155,7 @@ struct alignas(64) SimDesc {
   // Agent slots: n_slots = n from agent_off in both layouts of the agent arrays. Home
   // layout: slot = id. Office layout (hours of day 8..15): first the workers (Normal and
   // Essential) of office 0, 1, ... (an agent's office is id % n_offices), each office's in
-  // id order, then every other agent (not working, hospital staff) in id order; the
+  // id order, then every other agent (not working, hospital staff) house by house; the
   // office_agent array maps slot -> id. Workers spend these hours in their office, the
   // others near their house, so both groups keep neighbours in neighbouring slots.
   uint32_t n_slots;
