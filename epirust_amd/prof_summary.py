@@ -87,11 +87,17 @@ def trace(path, command, trace_csv=None, hours=0):
     rows = list(csv.DictReader(open(path)))
     out = ["# Kernel trace summary", "", "Command: `%s`" % command, "",
            "| kernel | calls | average µs | min µs | max µs | total ms | share |", "|---|---|---|---|---|---|---|"]
-    total = sum(float(r["TotalDurationNs"]) for r in rows)
-    for r in sorted(rows, key=lambda r: -float(r["TotalDurationNs"])):
+    per = {}  # a kernel's template instances together
+    for r in rows:
+        k = per.setdefault(short(r["Name"]), [0, 0.0, float("inf"), 0.0])
+        k[0] += int(r["Calls"])
+        k[1] += float(r["TotalDurationNs"])
+        k[2] = min(k[2], float(r["MinNs"]))
+        k[3] = max(k[3], float(r["MaxNs"]))
+    total = sum(k[1] for k in per.values())
+    for name, (calls, ns, lo, hi) in sorted(per.items(), key=lambda e: -e[1][1]):
         out.append("| %s | %s | %.2f | %.2f | %.2f | %.3f | %.1f%% |" % (
-            short(r["Name"]), r["Calls"], float(r["AverageNs"]) / 1e3, float(r["MinNs"]) / 1e3,
-            float(r["MaxNs"]) / 1e3, float(r["TotalDurationNs"]) / 1e6, 100.0 * float(r["TotalDurationNs"]) / total))
+            name, calls, ns / calls / 1e3, lo / 1e3, hi / 1e3, ns / 1e6, 100.0 * ns / total))
     text = "\n".join(out) + "\n"
     if trace_csv:
         text += "\n## By hour of day (first %d simulated hours)\n\n" % hours + by_hour_of_day(trace_csv, hours)
