@@ -370,15 +370,15 @@ int build_launch_tables(epi_sim* s) {
   return EPI_OK;
 }
 
-// The office layout's slot order (model.hpp): per simulation, the Normal and Essential
-// workers office by office (office = id % n_offices), each office's in id order, then the
-// other agents house by house. Work statuses are fixed at creation, so the slot maps are
-// built once, on the device from the synthesized state words, with the layout move's tiles.
 // Most agents of a handle whose office hours need no office layout: its two moves a day cost more
 // launches than its neighbours save (an hour of 20k agents 7.13 us with it, 6.83 without; of 40k
 // 7.08 and 7.27).
 constexpr uint64_t kHomeAgents = 30000;
 
+// The office layout's slot order (model.hpp): per simulation, the Normal and Essential
+// workers office by office (office = id % n_offices), each office's in id order, then the
+// other agents house by house. Work statuses are fixed at creation, so the slot maps are
+// built once, on the device from the synthesized state words, with the layout move's tiles.
 int build_office_order(epi_sim* s) {
   std::vector<OfficeJob> jobs;
   for (uint32_t i = 0; i < s->n_sims; ++i) {
@@ -397,7 +397,7 @@ int build_office_order(epi_sim* s) {
     for (uint32_t c : s->office_workers[i]) D.n_workers += c;
     // Tiles column by column (32 offices, every k), so that consecutive tiles share the
     // cache lines of their office slots: an office's workers, split over a column's k
-    // tiles, and the other agents of neighbouring columns, whose slots follow id order.
+    // tiles, and the other agents of neighbouring columns, who live in neighbouring houses.
     const uint32_t K = (n + O - 1u) / O;  // rows k of ids k * O + j
     for (uint32_t j0 = 0; j0 < O; j0 += 32)
       for (uint32_t k0 = 0; k0 < K; k0 += 32) tiles.push_back(TileRef{i, k0, j0});
@@ -433,11 +433,11 @@ int upload_tables(epi_sim* s) {
   return EPI_OK;
 }
 
-// Copies the agent arrays into the other layout.
 // Whether the agent arrays are in the office layout after `hour`, unless that ran in a home day's
 // graph, which ends in the home layout anyway.
 bool in_office_layout(const epi_sim* s, uint32_t hour) { return office_hour(hour) && !s->home_only; }
 
+// Copies the agent arrays into the other layout.
 int relayout(epi_sim* s, bool to_office) {
   HIP_TRY(launch_relayout(s->v, s->v_office, s->d_tiles, s->n_tiles, to_office, s->stream));
   return EPI_OK;

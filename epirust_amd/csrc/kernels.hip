@@ -29,6 +29,8 @@
 //              office's cells among the block's workers in LDS, and the winners on
 //              offices that lie wholly in one block (all of them when an office fits a
 //              block) claim nothing globally.
+//              Small handles, and days on which most agents are isolated, stay in the home
+//              layout throughout.
 //   k_night / k_quiet_hours: in day graphs, hours of day 1..6 (or 3..6) as one launch
 //              when no sweep can be pending inside them (no vaccination there).
 // A sweep decided at hour h (allocation_map.rs:306-337) is applied by the agent pass of
@@ -1043,8 +1045,8 @@ __global__ void k_hospital_scan(DevView v, uint32_t items_per_thread) {
 // Layout move of st and pos (tm and wsa, which few agents read, stay in the home layout and
 // are indexed by id in both), one tile of 32 x 32 agents id = k * n_offices + j per block.
 // Along j the ids are consecutive: the home side and the slot map are read (or written)
-// 128 B at a time, and so are the office slots of the tile's other agents, which keep id
-// order. Along k lie the workers of one office, which hold consecutive office slots: the
+// 128 B at a time; the office slots of the tile's other agents, who lie house by house, are
+// as close together as a house's agents are few. Along k lie the workers of one office, which hold consecutive office slots: the
 // workers go through LDS rows of 33 words so that their office side is also accessed a
 // column of the tile at a time. Each thread owns four rows of the tile and issues the loads
 // of all four before any store, so that a wave keeps four times the bytes in flight.
