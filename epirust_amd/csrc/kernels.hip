@@ -930,6 +930,12 @@ __global__ __attribute__((amdgpu_waves_per_eu(8))) void k_commit(const AgentBloc
   const SimDesc& D = desc[sim];
   const SimState* S = state + sim;
   uint32_t h = scalar_copy(&S->commit_hour[parity]);
+  // The movers' part of the descriptor comes while the agent words are in flight, not after them
+  // (an hour of 32 runs of 100k agents 39.01 -> 38.74 us, 10M 121.6 -> 121.2, 1M 17.17 -> 17.12).
+  uint64_t cell_off = scalar_copy(&D.cell_off), grid_off = scalar_copy(&D.grid_off);
+  uint32_t pitch = scalar_copy(&D.pitch), strip = scalar_copy(&D.strip);
+  const DiseaseParams dz = scalar_copy(&D.dz);
+  asm("" : "+s"(cell_off), "+s"(grid_off), "+s"(pitch), "+s"(strip), "+s"(h));
   loaded_together(m1, m2, m3);
   loaded_together(w, p, t, h);
   if (h == 0) return;  // uniform: the simulation did not step this hour
@@ -940,11 +946,7 @@ __global__ __attribute__((amdgpu_waves_per_eu(8))) void k_commit(const AgentBloc
   if (threadIdx.x < count) {
     const bool mover = t != kTgtNone;
     if (mover || (w & F_DIRTY)) {
-      const uint64_t cell_off = scalar_copy(&D.cell_off);
-      const uint32_t pitch = scalar_copy(&D.pitch);
-      const DiseaseParams dz = scalar_copy(&D.dz);
-      const uint32_t strip = scalar_copy(&D.strip);
-      uint8_t* occ = v.occ + scalar_copy(&D.grid_off);
+      uint8_t* occ = v.occ + grid_off;
       const uint8_t byte = occupant_byte(dz, w);
       bool moved = false;
       if (mover) {
