@@ -1007,12 +1007,15 @@ __global__ void k_hospital_scan(DevView v, uint32_t items_per_thread) {
   const uint32_t lead = static_cast<uint32_t>(hr.x0) + kPadX - strip0 * kStripStep;  // of the first item, before the area
   const uint32_t row0 = first / per_row, item0 = first - row0 * per_row;
   const uint32_t cell0 = row0 * wd + (item0 ? item0 * kStripStep - lead : 0u);  // the block's first cell
-  if (__hip_atomic_load(&S->first_vacant, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < cell0)
-    return;  // an earlier block already found one
+  // Whether an earlier block already found one. Other blocks lower the word in the meantime, so each
+  // wave may see its own answer: it decides only what that wave scans, and every wave writes its
+  // result and reaches the barrier.
+  const bool found_before =
+      __hip_atomic_load(&S->first_vacant, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < cell0;
   const uint8_t* occ = v.occ + D.grid_off;
   const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, waves = blockDim.x / kWave;
   uint32_t best = ~0u;
-  for (uint32_t k = 0; k < items_per_thread && best == ~0u; ++k) {  // uniform over the wave
+  for (uint32_t k = 0; k < items_per_thread && best == ~0u && !found_before; ++k) {  // uniform over the wave
     const uint32_t q = first + (k * waves + wave) * kWave + lane;
     const uint32_t row = q / per_row, item = q - row * per_row;
     uint32_t mine = ~0u;
