@@ -1479,23 +1479,23 @@ static int set_launch_blocks(epi_sim* sim, uint32_t home, uint32_t office) {
   if (office < 64 || office > 1024 || office % 64 || home < 64 || home > 1024 || home % 64)
     return fail(EPI_ERR_ARG, "block size must be 64..1024, x64");
   HIP_TRY(hipStreamSynchronize(sim->stream));
+  if (sim->home_only) {  // the caller chooses the office layout's blocks
+    const int rc = build_office_order(sim);
+    if (rc != EPI_OK) return rc;  // nothing that a launch reads has changed
+  }
+  const LaunchShape before = sim->shape;
   sim->shape.block = home;
   sim->shape.office_block = office;
-  const bool leaves_home = sim->home_only;
-  int rc = EPI_OK;
-  if (leaves_home) {  // the caller chooses the office layout's blocks
-    rc = build_office_order(sim);
-    if (rc != EPI_OK) return rc;
-    sim->home_only = false;
+  int rc = build_launch_tables(sim);
+  if (rc == EPI_OK) rc = upload_tables(sim);
+  if (rc == EPI_OK && sim->home_only && sim->host_hour > 0 && office_hour(sim->host_hour)) rc = relayout(sim, true);
+  if (rc != EPI_OK) {  // the launches' threads have to be those of their tables
+    const std::string why = g_last_error;
+    sim->shape = before;
+    if (build_launch_tables(sim) == EPI_OK) (void)upload_tables(sim);
+    return fail(rc, why);
   }
-  rc = build_launch_tables(sim);
-  if (rc != EPI_OK) return rc;
-  rc = upload_tables(sim);
-  if (rc != EPI_OK) return rc;
-  if (leaves_home && sim->host_hour > 0 && office_hour(sim->host_hour)) {
-    rc = relayout(sim, true);
-    if (rc != EPI_OK) return rc;
-  }
+  sim->home_only = false;
   for (hipGraphExec_t* graphs : {sim->day_graph, sim->days_graph})
     for (uint32_t f = 0; f < DAY_VARIANTS; ++f)
       if (graphs[f]) {

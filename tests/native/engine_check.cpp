@@ -1,0 +1,66 @@
+// The host runtime (epirust_amd/csrc/engine.cpp) on a device played on the host: one check per run,
+// named by the first argument.
+#include "fake_device.hpp"
+
+static std::string config(uint32_t agents, uint32_t grid, uint32_t hours, const std::string& interventions) {
+  return "{\"population\":{\"Auto\":{\"number_of_agents\":" + std::to_string(agents) +
+         ",\"public_transport_percentage\":0.2,\"working_percentage\":0.7}},"
+         "\"disease\":{\"regular_transmission_start_day\":5,\"high_transmission_start_day\":20,\"last_day\":23,"
+         "\"asymptomatic_last_day\":9,\"mild_infected_last_day\":12,\"regular_transmission_rate\":0.025,"
+         "\"high_transmission_rate\":0.25,\"death_rate\":0.2,\"percentage_asymptomatic_population\":0.3,"
+         "\"percentage_severe_infected_population\":0.3,\"exposed_duration\":48,\"pre_symptomatic_duration\":48},"
+         "\"geography_parameters\":{\"grid_size\":" + std::to_string(grid) + ",\"hospital_beds_percentage\":0.003},"
+         "\"hours\":" + std::to_string(hours) + ",\"interventions\":[" + interventions + "],"
+         "\"starting_infections\":{\"exposed\":20,\"infected_mild_asymptomatic\":0,\"infected_mild_symptomatic\":0,"
+         "\"infected_severe\":0}}";
+}
+#define EXPECT(x)                                                              \
+  do {                                                                         \
+    if (!(x)) {                                                                \
+      std::printf("line %d: %s (%s)\n", __LINE__, #x, epi_last_error());       \
+      std::exit(1);                                                            \
+    }                                                                          \
+  } while (0)
+
+static epi_sim* create(uint32_t agents, uint32_t grid, uint32_t hours, const std::string& interventions = "") {
+  epi_sim* sim = nullptr;
+  EXPECT(epi_create(config(agents, grid, hours, interventions).c_str(), 1, 0, &sim) == EPI_OK);
+  fake.launches.clear();
+  fake.captures = 0;
+  return sim;
+}
+static uint32_t step(epi_sim* sim, uint32_t hours, int* stopped = nullptr) {
+  std::vector<epi_counts> rows(hours);
+  uint32_t n = 0;
+  int stop = 0;
+  EXPECT(epi_step(sim, hours, rows.data(), &n, &stop) == EPI_OK);
+  if (stopped) *stopped = stop;
+  return n;
+}
+
+// A block size that cannot be set leaves the handle as it was.
+static void block_size_failure() {
+  for (uint32_t agents : {2000u, 40000u}) {  // without and with an office layout
+    for (int copies = -1; copies < 3; ++copies) {
+      if (copies < 0 && agents > 30000u) continue;
+      epi_sim* sim = create(agents, agents / 20u, 2400);
+      EXPECT(step(sim, 34) == 34);  // ends in office hours
+      fake.maps_fail = copies < 0;
+      fake.copies_before_failure = copies;
+      EXPECT(epi_set_block_size(sim, 64) == EPI_ERR_DEVICE);
+      fake.maps_fail = false;
+      fake.copies_before_failure = -1;
+      EXPECT(step(sim, 100) == 100 && !fake.wrong_blocks);
+      EXPECT(epi_set_block_size(sim, 1024) == EPI_OK);
+      EXPECT(step(sim, 100) == 100 && !fake.wrong_blocks);
+      epi_destroy(sim);
+    }
+  }
+}
+
+int main(int, char** argv) {
+  const std::string check = argv[1];
+  if (check == "block_size_failure") block_size_failure();
+  else return 2;
+  std::puts("ok");
+}
