@@ -408,7 +408,7 @@ def main():
                    "kernel_ms": {"hospital_scan": scan_ms, "step": step_ms, "commit": commit_ms}},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": "one simulated hour: k_commit with its folded epilogue every hour, k_step at hours of day 0 and 7..23, k_hospital_scan once a day",
+                     "kernel": "one simulated hour: k_step and k_commit with its folded epilogue at hours of day 0 and 7..23, k_night for hours 1..6 together, k_hospital_scan once a day",
                      "basis": "HIP events on the handle's stream around the timed hour loop: %.2f us of device time per simulated hour" % hour_us,
                      "algorithmic_bytes_per_hour": algorithmic_bytes_per_hour(n, g)},
     }

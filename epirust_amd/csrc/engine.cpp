@@ -469,7 +469,11 @@ int enqueue_hour(epi_sim* s, uint32_t next_hour, bool home_day = false) {
     if (rc != EPI_OK) return rc;
   }
   const DevView& v = office_hour(next_hour) && !home_day ? s->v_office : s->v;
-  if (hour_has_step(next_hour)) HIP_TRY(launch_step(v, s->shape, next_hour, s->stream));
+  if (!hour_has_step(next_hour)) {
+    HIP_TRY(launch_rest(v, s->shape, next_hour, s->stream));
+    return EPI_OK;
+  }
+  HIP_TRY(launch_step(v, s->shape, next_hour, s->stream));
   HIP_TRY(launch_commit(v, s->shape, next_hour, s->stream));
   return EPI_OK;
 }
@@ -1432,7 +1436,8 @@ int epi_profile(epi_sim* sim, uint32_t n_hours, double ms_mean[3], uint32_t laun
       const DevView& v = in_office_layout(sim, h) ? sim->v_office : sim->v;
       if (had_step[k] && launch_step(v, sim->shape, h, sim->stream) != hipSuccess) rc = fail(EPI_ERR_DEVICE, "launch");
       (void)hipEventRecord(e[2], sim->stream);
-      if (launch_commit(v, sim->shape, h, sim->stream) != hipSuccess) rc = fail(EPI_ERR_DEVICE, "launch");
+      if ((had_step[k] ? launch_commit : launch_rest)(v, sim->shape, h, sim->stream) != hipSuccess)
+        rc = fail(EPI_ERR_DEVICE, "launch");
       (void)hipEventRecord(e[3], sim->stream);
       ++sim->host_hour;
     }

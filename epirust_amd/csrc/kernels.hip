@@ -10,18 +10,19 @@
 //              32-bit atomicMin keyed (claim hour, agent id) unless the office filter or
 //              housemate arbitration settles it; S/E/I/H/R/D counted with wavefront
 //              ballots into per-block partials.
-//   k_commit : every hour. Its first blocks, one per simulation, run the hour's epilogue:
+//   k_commit : hours of day 0 and 7..23. Its first blocks, one per simulation, run the epilogue:
 //              reduce the partials, write the row, run the intervention triggers and the
 //              stop rule on device; the row and the state go to device memory and to the
 //              host's pinned copies, which a step call reads after its one drain. The other
 //              blocks run the hour's agent pass, which
 //              reads nothing the same hour's epilogue writes (its hour and its sweep come
 //              from parity slots the previous epilogue filled), so the two share a launch.
-//              At hours of day 0 and 7..23 the agent pass commits the moves (the claim
-//              winner moves, grid bytes are updated). Hours of day 1..6 move nobody and
-//              change no state but flags and areas (citizen/mod.rs:244-248): the epilogue
-//              repeats the last counts and the agent pass applies the pending sweep, sets
-//              non-staff areas to home at hour of day 1 and resets the claim array at 2.
+//              The agent pass commits the moves (the claim winner moves, grid bytes are
+//              updated).
+//   k_rest   : hours of day 1..6, which move nobody and change no state but flags and areas
+//              (citizen/mod.rs:244-248): the epilogue repeats the last counts and the agent
+//              pass applies the pending sweep, sets non-staff areas to home at hour of day 1
+//              and resets the claim array at 2.
 //   k_relayout: [hours of day 8 and 16] moves st and pos between the home layout
 //              (slot = agent id) and the office layout that hours of day 8..15 run on:
 //              each office's workers in consecutive slots, packed whole into blocks,
@@ -591,9 +592,8 @@ __device__ __forceinline__ void add_partials(uint32_t (&acc)[6], const uint32_t*
   }
 }
 
-// The hour's epilogue of simulation `sim` by one block: adds up the hour's per-block partial
-// counts (hours of day 1..6 repeat the last counts: nobody's state changes), then
-// hour_epilogue on thread 0, whose other inputs are loaded first so they arrive with the
+// The epilogue of an hour of day 0 or 7..23 of simulation `sim` by one block: adds up the hour's
+// per-block partial counts, then hour_epilogue on thread 0, whose other inputs are loaded first so they arrive with the
 // partials. At up to 100k agents the commit is as long as this block, a chain of latencies:
 // descriptor and state once by scalar loads, the counts in two wide loads per block, sums by
 // DPP and one barrier; the state is worked on in registers and written once. With the step's
@@ -613,26 +613,18 @@ __device__ __forceinline__ void epilogue_block(const DevView& v, const SimDesc* 
     return;
   }
   const uint32_t h = in.st.hour + 1u;
-  uint32_t c[6];
-  if (h % 24u >= 1 && h % 24u <= 6) {  // uniform
+  uint32_t acc[6] = {0, 0, 0, 0, 0, 0}, c[6] = {0, 0, 0, 0, 0, 0};
+  add_partials(acc, v.block_counts + 8ull * (ONE ? 0u : in.D.block_begin), in.D.n_blocks);
+  // Each wave's six sums to its own LDS words, then thread 0 adds up the waves'.
 #pragma unroll
-    for (int k = 0; k < 6; ++k) c[k] = in.st.last_counts[k];
-  } else {
-    uint32_t acc[6] = {0, 0, 0, 0, 0, 0};
-    add_partials(acc, v.block_counts + 8ull * (ONE ? 0u : in.D.block_begin), in.D.n_blocks);
-    // Each wave's six sums to its own LDS words, then thread 0 adds up the waves'.
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      const uint32_t x = wave_sum(acc[k]);
-      if ((threadIdx.x & (kWave - 1)) == kWave - 1) s_sum[threadIdx.x / kWave][k] = x;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 6; ++k) c[k] = 0;
-    for (uint32_t q = 0; q < blockDim.x / kWave; ++q)
-#pragma unroll
-      for (int k = 0; k < 6; ++k) c[k] += s_sum[q][k];
+  for (int k = 0; k < 6; ++k) {
+    const uint32_t x = wave_sum(acc[k]);
+    if ((threadIdx.x & (kWave - 1)) == kWave - 1) s_sum[threadIdx.x / kWave][k] = x;
   }
+  __syncthreads();
+  for (uint32_t q = 0; q < blockDim.x / kWave; ++q)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) c[k] += s_sum[q][k];
   if (threadIdx.x == 0) {
     hour_epilogue(v, in, h, c);
     store_state(v, sim, in);
@@ -806,11 +798,8 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_step(const AgentBlock* bl
   }
 }
 
-// Epilogues of hours of day 3..6 in one launch (one block per simulation, thread 0 walks
-// the hours), for day graphs of simulations with no vaccination at hours of day 2..5. Then
-// no sweep is pending at any of those hours (lockdown, unlock and hospital decisions fall
-// on hours of day 0 only), so their agent passes would change nothing. Each hour does
-// what epilogue_block does for it.
+// Epilogues of hours of day 1..6 (thread 0 of a block walks the hours): nobody's state changes
+// then, so each repeats the last counts.
 __device__ void quiet_epilogues(const DevView& v, uint32_t sim, uint32_t n_hours) {
   EpilogueIn in;
   load_epilogue_in(v, v.desc, v.state, sim, in);
@@ -826,6 +815,9 @@ __device__ void quiet_epilogues(const DevView& v, uint32_t sim, uint32_t n_hours
   }
   store_state(v, sim, in);
 }
+// Hours of day 3..6 in one launch, one block per simulation, for days with no vaccination at
+// hours of day 2..5. Then no sweep is pending at any of those hours (lockdown, unlock and hospital
+// decisions fall on hours of day 0 only), so their agent passes would change nothing.
 __global__ void k_quiet_hours(DevView v, uint32_t n_hours) {
   if (threadIdx.x == 0) quiet_epilogues(v, blockIdx.x, n_hours);
 }
@@ -862,16 +854,29 @@ __global__ __attribute__((amdgpu_num_sgpr(80))) void k_night(DevView v, uint32_t
   reset_claims(share);
 }
 
-// Agent pass of an hour of day 1..6 (block b of the simulation's agent blocks): nobody
-// moves and no disease update runs while asleep (citizen/mod.rs:244-248), so only the
-// sweep decided at hour h - 1 is applied, hour of day 1 sets every non-staff current area
-// to home, and hour of day 2 resets the claim array before the day's first claim hour.
-__device__ __forceinline__ void rest_pass(const DevView& v, const SimDesc& D, const SimState& S, uint32_t h,
-                                          uint32_t local, uint32_t b) {
-  const uint32_t hd = h % 24u;
-  const Sweep sweep = sweep_slot(S, (h - 1u) & 1u);
+// One hour of day 1..6 (home layout). Blocks 0 .. n_epi-1 run the epilogue of simulation
+// blockIdx.x; the rest its agent work: nobody moves and no disease update runs while asleep
+// (citizen/mod.rs:244-248), so only the sweep decided at hour h - 1 is applied, hour of day 1 sets
+// every non-staff current area to home, and hour of day 2 resets the claim array before the day's
+// first claim hour. A kernel of its own, whose blocks read the agents only where one of these asks
+// for them (hours of day 1, 2 and 3..6 of 10M agents as a branch of the commit behind its loads 47,
+// 62 and 30 us; so 27, 30 and 15-16, which is the time to start 19,500 blocks).
+__global__ __attribute__((amdgpu_num_sgpr(80))) void k_rest(DevView v, uint32_t parity, uint32_t n_epi) {
+  if (blockIdx.x < n_epi) {  // uniform
+    if (threadIdx.x == 0) quiet_epilogues(v, blockIdx.x, 1);
+    return;
+  }
+  const uint32_t b = blockIdx.x - n_epi;
+  const AgentBlock bm = scalar_copy(v.agent_blocks + b);
+  const uint32_t sim = first_lane(bm.sim);
+  const SimDesc& D = v.desc[sim];
+  const SimState* S = v.state + sim;
+  const uint32_t h = S->commit_hour[parity];
+  if (h == 0) return;  // uniform: the simulation did not step this hour
+  const uint32_t hd = h % 24u, local = first_lane(bm.first) + threadIdx.x;
+  const Sweep sweep = sweep_slot(*S, (h - 1u) & 1u);
   ClaimShare share{nullptr, 0, 0};
-  if (hd == 2) share = claim_share(v, D, b);
+  if (hd == 2) share = claim_share(v, D, b - D.block_begin);
   if (local < D.n && (sweep.mask || hd == 1)) {
     const uint64_t gi = D.agent_off + local;
     const uint32_t w = v.st[gi];
@@ -889,9 +894,9 @@ __device__ __forceinline__ void put_byte(uint8_t* occ, uint32_t strip, uint32_t 
   if (in_two_strips(g)) occ[second_place(strip, g)] = byte;
 }
 
-// `parity` is the hour's parity (an hour of day 24k + j has the parity of j). Blocks
-// 0 .. n_epi-1 run the epilogue of simulation blockIdx.x; the rest run the agent pass:
-// the commit at hours of day 0 and 7..23, rest_pass at 1..6. Eight waves per SIMD (64 VGPRs)
+// The commit of an hour of day 0 or 7..23. `parity` is the hour's parity (an hour of day 24k + j
+// has the parity of j). Blocks 0 .. n_epi-1 run the epilogue of simulation blockIdx.x; the rest
+// run the agent pass. Eight waves per SIMD (64 VGPRs)
 // for the agent pass, whose waves mostly wait for the grid: with the 98 VGPRs that the
 // epilogue would take, an hour of 10M agents takes 177 us instead of 160.
 // Arguments and ONE as in k_step.
@@ -939,10 +944,6 @@ __global__ __attribute__((amdgpu_waves_per_eu(8))) void k_commit(const AgentBloc
   loaded_together(m1, m2, m3);
   loaded_together(w, p, t, h);
   if (h == 0) return;  // uniform: the simulation did not step this hour
-  if (h % 24u >= 1 && h % 24u <= 6) {  // uniform; home layout
-    rest_pass(v, D, *S, h, first_lane(bm.first) + threadIdx.x, blockIdx.x - (ONE ? 1u : n_epi) - D.block_begin);
-    return;
-  }
   if (threadIdx.x < count) {
     const bool mover = t != kTgtNone;
     if (mover || (w & F_DIRTY)) {
@@ -1197,6 +1198,12 @@ hipError_t launch_commit(const DevView& v, const LaunchShape& s, uint32_t hour, 
   const auto kernel = s.n_sims == 1 ? k_commit<true> : k_commit<false>;
   hipLaunchKernelGGL(kernel, dim3(s.n_sims + blocks), dim3(v.office ? s.office_block : s.block), 0, stream,
                      v.agent_blocks, v.desc, v.state, v.st, v.pos, v.tgt, hour & 1u, s.n_sims, v);
+  return hipGetLastError();
+}
+
+hipError_t launch_rest(const DevView& v, const LaunchShape& s, uint32_t hour, hipStream_t stream) {
+  if (s.agent_blocks + s.n_sims == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_rest, dim3(s.n_sims + s.agent_blocks), dim3(s.block), 0, stream, v, hour & 1u, s.n_sims);
   return hipGetLastError();
 }
 

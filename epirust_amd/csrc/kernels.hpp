@@ -54,13 +54,14 @@ struct LaunchShape {
   uint32_t n_sims = 0;
 };
 
-// One hour: [hour of day 0] scan, [hours of day 0 and 7..23] step, then the commit launch:
-// the epilogue in its first blocks and the hour's agent pass in the rest (the commit at
-// hours of day 0 and 7..23, the pending sweep / area reset / claim reset at 1..6).
+// One hour of day 0 or 7..23: [hour of day 0] scan, step, then the commit launch, the epilogue in
+// its first blocks and the commit of the moves in the rest. One of 1..6: the rest launch, the
+// epilogue and the pending sweep / area reset / claim reset (home layout).
 // `hour` only needs the right hour of day, so a captured day of hours 1..24 replays for any day.
 hipError_t launch_hospital_scan(const DevView& v, const LaunchShape& s, hipStream_t stream);
 hipError_t launch_step(const DevView& v, const LaunchShape& s, uint32_t hour, hipStream_t stream);
 hipError_t launch_commit(const DevView& v, const LaunchShape& s, uint32_t hour, hipStream_t stream);
+hipError_t launch_rest(const DevView& v, const LaunchShape& s, uint32_t hour, hipStream_t stream);
 // Copies st and pos between the home and office layouts (to_office: home -> office), one
 // 32 x 32 tile of (k, j) per block.
 hipError_t launch_relayout(const DevView& home, const DevView& office, const TileRef* tiles, uint32_t n_tiles,

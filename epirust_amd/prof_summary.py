@@ -21,9 +21,9 @@ import json
 import re
 import sys
 
-HOUR_KERNELS = ("k_hospital_scan", "k_relayout", "k_step", "k_commit", "k_quiet_hours", "k_night")
-# dispatches that close several hours: k_quiet_hours runs hours of day 3..6, k_night 1..6
-SPAN = {"k_commit": 1, "k_quiet_hours": 4, "k_night": 6}
+HOUR_KERNELS = ("k_hospital_scan", "k_relayout", "k_step", "k_commit", "k_rest", "k_quiet_hours", "k_night")
+# hours that a dispatch closes: k_quiet_hours runs hours of day 3..6, k_night 1..6
+SPAN = {"k_commit": 1, "k_rest": 1, "k_quiet_hours": 4, "k_night": 6}
 
 
 def short(name):
@@ -37,8 +37,8 @@ def short(name):
 
 def by_hour_of_day(trace_csv, hours):
     """Mean duration per kernel for each hour of day over the first `hours` hours of the
-    trace (an hour is [k_hospital_scan] [k_relayout] [k_step] k_commit: hours are counted by
-    k_commit dispatches; a k_quiet_hours dispatch stands for the four hours of day 3..6 and
+    trace (an hour is [k_hospital_scan] [k_relayout] k_step k_commit, or k_rest at hours of day
+    1..6: hours are counted by k_commit and k_rest dispatches; a k_quiet_hours dispatch stands for the four hours of day 3..6 and
     a k_night dispatch for the six of 1..6, reported at their first hour), with the wall
     time from one hour's first kernel to the next hour's (a dispatch that closes several
     hours has its wall time split evenly over them)."""
@@ -195,7 +195,7 @@ def counters(paths, command, clock_ghz=2.4):
 def hourly(paths, command):
     """Per hour of day, the mean per dispatch of each counter of k_step and k_commit, from
     counter_collection.csv files of `bench.py --profile-hours H` (every hour dispatched on
-    its own; hours are counted by k_commit dispatches), with the L2 hit rate where
+    its own; hours are counted by k_commit and k_rest dispatches), with the L2 hit rate where
     TCC_HIT / TCC_MISS are present."""
     per = collections.defaultdict(lambda: collections.defaultdict(lambda: collections.defaultdict(list)))
     names = set()
@@ -212,7 +212,7 @@ def hourly(paths, command):
                 for c, v in vals.items():
                     per[hour % 24][k][c].append(v)
                     names.add(c)
-            if k == "k_commit":
+            if k in ("k_commit", "k_rest"):
                 hour += 1
     names = sorted(names)
     hit = "TCC_HIT_sum" in names and "TCC_MISS_sum" in names

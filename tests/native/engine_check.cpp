@@ -58,9 +58,31 @@ static void block_size_failure() {
   }
 }
 
+// Hours of day 1..6 launch the kernel that reads the agents only where a sweep, hour 1 or 2 asks for
+// it, hour at a time, in calls that end inside a day, without graphs and in a profile.
+static void rest_hours() {
+  for (uint32_t flags : {0u, (unsigned)EPI_FLAG_NO_GRAPH}) {
+    for (uint32_t call : {1u, 2u, 5u, 24u}) {
+      epi_sim* sim = nullptr;
+      EXPECT(epi_create(config(2000, 100, 2400, "").c_str(), 1, flags, &sim) == EPI_OK);
+      fake.launches.clear();
+      for (uint32_t h = 0; h < 240; h += call) EXPECT(step(sim, call) == call);
+      EXPECT(fake.count("commit") == 240 / 24 * 18 && fake.count("step") == 240 / 24 * 18);
+      if (call <= 2 || flags) EXPECT(fake.count("rest") == 240 / 24 * 6);
+      fake.launches.clear();
+      double ms[3];
+      uint32_t launches[3], hours = 0;
+      EXPECT(epi_profile(sim, 48, ms, launches, &hours) == EPI_OK && hours == 48);
+      EXPECT(fake.count("commit") == 36 && fake.count("rest") == 12);
+      epi_destroy(sim);
+    }
+  }
+}
+
 int main(int, char** argv) {
   const std::string check = argv[1];
   if (check == "block_size_failure") block_size_failure();
+  else if (check == "rest_hours") rest_hours();
   else return 2;
   std::puts("ok");
 }

@@ -178,6 +178,9 @@ hipError_t launch_step(const DevView& v, const LaunchShape& s, uint32_t, hipStre
 hipError_t launch_commit(const DevView& v, const LaunchShape& s, uint32_t, hipStream_t) {
   return over_agents("commit", v, s, [=] { fake_epilogues(v, s, 1); }), hipSuccess;
 }
+hipError_t launch_rest(const DevView& v, const LaunchShape& s, uint32_t, hipStream_t) {
+  return over_agents("rest", v, s, [=] { fake_epilogues(v, s, 1); }), hipSuccess;
+}
 hipError_t launch_night(const DevView& v, const LaunchShape& s, hipStream_t) {
   return over_agents("night", v, s, [=] { fake_epilogues(v, s, 6); }), hipSuccess;
 }

@@ -99,3 +99,23 @@ def test_hourly_counters_follow_the_commit_count(tmp_path):
     assert table[(9, "k_commit")] == (910.5, 2732.0, "25%")
     assert table[(0, "k_step")] == (0.5, 1.5, "25%")
     assert (3, "k_commit") not in table  # only hours of day 7..23 and 0 are listed
+
+
+def test_rest_launches_count_as_hours(tmp_path):
+    """Hours of day 1..6 that run one by one are k_rest dispatches."""
+    p = tmp_path / "r.csv"
+    one = [("k_rest", 6000)] + [("k_rest", 3000)] * 5 + day("night")[1:]
+    write_trace(p, one + one)
+    r = rows(P.by_hour_of_day(str(p), 48))
+    cols = list(P.HOUR_KERNELS)
+    assert r[1][cols.index("k_rest")] == 6.0 and all(r[hd][cols.index("k_rest")] == 3.0 for hd in (2, 3, 4, 5, 6))
+    assert r[7][cols.index("k_step")] == 20.0 and r[0][cols.index("k_commit")] == 10.0
+    assert all(r[hd][cols.index("k_rest")] == 0.0 for hd in (0, 7, 23))
+    path = tmp_path / "counters.csv"
+    with open(path, "w", newline="") as f:
+        w = csv.DictWriter(f, fieldnames=["Dispatch_Id", "Kernel_Name", "Counter_Name", "Counter_Value"])
+        w.writeheader()
+        for d, k in enumerate(["k_rest"] * 6 + ["k_step", "k_commit"] * 18):
+            w.writerow({"Dispatch_Id": d, "Kernel_Name": NAME % k, "Counter_Name": "SQ_WAVES", "Counter_Value": d})
+    lines = P.hourly([str(path)], "cmd").splitlines()
+    assert "| 7 | k_step | 6 |" in lines and "| 0 | k_commit | 41 |" in lines
