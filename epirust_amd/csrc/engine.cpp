@@ -491,18 +491,34 @@ bool mostly_isolated(const epi_sim* s) {
   return 2.0 * isolated >= static_cast<double>(s->n_agents) && s->n_agents != 0;
 }
 
+// Whether some simulation cannot stop before `hour`, by the states that the host has so far: it has
+// someone exposed, who is infected for nine days at least (disease.hpp; a severe case for last_day).
+// Another disease handler may be quicker: then days are enqueued that find the run stopped.
+bool runs_until(const epi_sim* s, uint32_t hour) {
+  for (uint32_t i = 0; i < s->n_sims; ++i) {
+    const volatile SimState& st = const_cast<const volatile SimState*>(s->pinned_state)[i];
+    if (st.active && st.last_counts[1] && st.hour + 24u * std::min(9u, s->cfg[i].last_day) >= hour) return true;
+  }
+  return false;
+}
+
 // Days of equal flags that one graph runs in handles of at most kGraphAgents: between two graphs
-// lie the active flags' export and its event, 6.5 us (an hour of 10k agents 6.50 us with a graph
-// per day, 6.22 with four days; 100k 7.40, 7.22; 1M 18.40, 18.12; 32 runs of 100k 40.35, 39.87).
-// Larger ones gain less than they lose to the later sight of a lockdown (mostly_isolated).
-constexpr uint32_t kGraphDays = 4;
+// lie the active flags' export and its event, 6.5 us (an hour of 10k agents 6.23 us with a graph
+// per day, 5.95 with four days; 100k 7.20, 6.94; 1M 17.40, 17.11; 32 runs of 100k 39.20, 38.66).
+// At 5M and 10M agents neither is faster (62.1, 62.0 and 135.6, 135.7), and with a lockdown, which is
+// seen later (mostly_isolated), four days are slower (63.1, 63.7 and 121.2, 121.5).
+// Only while the run is known to go on that long, as a stop is seen two graphs late and an empty
+// day takes 65 us; and not in its first days, as a run whose starting infections die out would
+// not win back the time to build the graph, 170 us (10k agents that nobody infects, 23 days:
+// four days throughout 4.20 ms, 3.88 so, a graph per day 3.87; 1M 7.04, 6.51, 6.49).
+constexpr uint32_t kGraphDays = 4, kFirstDays = 8;
 constexpr uint64_t kGraphAgents = 4000000;
 uint32_t graph_days(const epi_sim* s, uint32_t target) {
-  if (s->n_agents > kGraphAgents || target - s->host_hour < 24u * kGraphDays) return 1;
+  if (s->n_agents > kGraphAgents || s->host_hour < 24u * kFirstDays || target - s->host_hour < 24u * kGraphDays) return 1;
   const uint8_t* flags = &s->day_flags[s->host_hour / 24u];
   for (uint32_t d = 1; d < kGraphDays; ++d)
     if (flags[d] != flags[0]) return 1;
-  return kGraphDays;
+  return runs_until(s, s->host_hour + 24u * kGraphDays) ? kGraphDays : 1;
 }
 
 // The groups of hours that the day from `hour` + 1 on runs as one launch each.

@@ -79,10 +79,40 @@ static void rest_hours() {
   }
 }
 
+// After a run has stopped no more than the rest of its day and one day more are launched, whichever
+// day it stops on; while somebody is exposed a graph runs four days.
+static void days_after_the_stop() {
+  for (uint32_t agents : {2000u, 40000u})
+    for (uint32_t stop = 24u * 9u; stop < 24u * 16u; stop += 13u) {
+      epi_sim* sim = create(agents, agents / 20u, 2400);
+      fake.stop_hour = stop;
+      fake.exposed_until = stop - 24u * 9u;  // ill for nine days at least
+      int stopped = 0;
+      EXPECT(step(sim, 2399, &stopped) == stop && stopped);
+      double ms = 0;
+      uint32_t hours = 0;
+      EXPECT(epi_last_run_ms(sim, &ms, &hours) == EPI_OK);
+      EXPECT(hours <= (stop + 23u) / 24u * 24u + 24u);
+      epi_destroy(sim);
+    }
+  fake.stop_hour = fake.exposed_until = ~0u;
+  epi_sim* sim = create(2000, 100, 2400);
+  fake.graphs = 0;
+  EXPECT(step(sim, 2399) == 2399 && fake.graphs <= 8u + 23u + 3u);
+  epi_destroy(sim);
+  // a run whose starting infections die out builds one graph only
+  fake.stop_hour = 500;
+  fake.exposed_until = 55;
+  sim = create(2000, 100, 2400);
+  EXPECT(step(sim, 2399) == 500 && fake.captures == 1);
+  epi_destroy(sim);
+}
+
 int main(int, char** argv) {
   const std::string check = argv[1];
   if (check == "block_size_failure") block_size_failure();
   else if (check == "rest_hours") rest_hours();
+  else if (check == "days_after_the_stop") days_after_the_stop();
   else return 2;
   std::puts("ok");
 }

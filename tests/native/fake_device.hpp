@@ -21,10 +21,11 @@
 struct Fake {
   uint32_t stop_hour = ~0u;  // nobody is ill any more from this hour on
   uint32_t lock_hour = ~0u;  // a lockdown comes at this hour
+  uint32_t exposed_until = 0;  // the last hour after which somebody is exposed
   bool maps_fail = false;    // building the office layout's slot maps fails
   int copies_before_failure = -1;  // of tables to the device, while it is not negative
   bool wrong_blocks = false;  // a launch whose threads per block are not its table's
-  uint32_t captures = 0;      // graphs instantiated
+  uint32_t captures = 0, graphs = 0;  // graphs instantiated, and launched
   std::vector<std::string> launches;  // kernels run, the idle ones of stopped runs as "idle"
   uint32_t count(const std::string& name) const {
     uint32_t n = 0;
@@ -99,6 +100,7 @@ hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, hipGraphNode_t*,
 hipError_t hipGraphDestroy(hipGraph_t g) { return delete reinterpret_cast<FakeGraph*>(g), hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t e) { return delete reinterpret_cast<FakeGraph*>(e), hipSuccess; }
 hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
+  ++fake.graphs;
   for (const Work& w : reinterpret_cast<FakeGraph*>(e)->nodes) enqueue(w);
   return hipSuccess;
 }
@@ -137,6 +139,7 @@ inline void fake_epilogues(const DevView& v, const LaunchShape& s, uint32_t hour
       const uint32_t h = ++st.hour;
       st.rows_written = h;
       v.rows[D.row_off + h - 1] = v.host_rows[D.row_off + h - 1] = Counts7{h, D.n, 0, 0, 0, 0, 0};
+      st.last_counts[1] = h <= fake.exposed_until;
       if (h == fake.lock_hour) st.locked = 1;
       if (h >= fake.stop_hour || h + 1 >= D.hours) st.active = 0;
       v.host_state[i] = st;
