@@ -482,8 +482,10 @@ int enqueue_hour(epi_sim* s, uint32_t next_hour, bool home_day = false) {
 // the host has so far (up to two graphs old while a call runs ahead). They stay where they are, so
 // the office layout's neighbours are not neighbours then (10M agents with a lockdown on day 22 of
 // 60: 144.3 us an hour on the office layout throughout, 134.5 with this rule, 172 on the home
-// layout throughout; 32 runs of 100k with one: 43.9, 40.8, 51.4). Either gives the same results.
+// layout throughout; 32 runs of 100k with one: 43.9, 40.8, 51.4). Either gives the same results. A
+// handle without an office layout has nothing to choose, and keeps the graphs that it has.
 bool mostly_isolated(const epi_sim* s) {
+  if (s->home_only) return false;
   double isolated = 0.0;
   for (uint32_t i = 0; i < s->n_sims; ++i)
     if (const_cast<const volatile SimState*>(s->pinned_state)[i].locked)

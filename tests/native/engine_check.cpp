@@ -108,11 +108,27 @@ static void days_after_the_stop() {
   epi_destroy(sim);
 }
 
+// A lockdown asks for other launches only of a handle with an office layout: the others replay the
+// graphs that they have.
+static void graphs_under_a_lockdown() {
+  const std::string lockdown = "{\"Lockdown\":{\"at_number_of_infections\":10,\"essential_workers_population\":0.1}}";
+  fake.exposed_until = ~0u;
+  for (uint32_t agents : {2000u, 40000u}) {
+    fake.lock_hour = 480;
+    epi_sim* sim = create(agents, agents / 20u, 2400, lockdown);
+    EXPECT(step(sim, 24u * 96u) == 24u * 96u);
+    EXPECT(fake.captures == (agents <= 30000u ? 2u : 3u));  // a day, four days, four home days
+    EXPECT((fake.count("relayout") == 0) == (agents <= 30000u));
+    epi_destroy(sim);
+  }
+}
+
 int main(int, char** argv) {
   const std::string check = argv[1];
   if (check == "block_size_failure") block_size_failure();
   else if (check == "rest_hours") rest_hours();
   else if (check == "days_after_the_stop") days_after_the_stop();
+  else if (check == "graphs_under_a_lockdown") graphs_under_a_lockdown();
   else return 2;
   std::puts("ok");
 }

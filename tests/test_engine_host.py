@@ -20,7 +20,8 @@ def checks(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["block_size_failure", "rest_hours", "days_after_the_stop"])
+@pytest.mark.parametrize("check", ["block_size_failure", "rest_hours", "days_after_the_stop",
+                                   "graphs_under_a_lockdown"])
 def test_engine(checks, check):
     out = subprocess.run([checks, check], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout + out.stderr
