@@ -123,12 +123,26 @@ static void graphs_under_a_lockdown() {
   }
 }
 
+// Small handles move to the office layout, twice a day, once their block size is set; larger ones have
+// it by themselves.
+static void small_handles_with_an_office_layout() {
+  for (uint32_t agents : {2000u, 30000u, 30001u})
+    for (bool set : {false, true}) {
+      epi_sim* sim = create(agents, 400, 2400);
+      if (set) EXPECT(epi_set_block_size(sim, 256) == EPI_OK);
+      EXPECT(step(sim, 240) == 240);
+      EXPECT(fake.count("relayout") == (set || agents > 30000u ? 20u : 0u) && !fake.wrong_blocks);
+      epi_destroy(sim);
+    }
+}
+
 int main(int, char** argv) {
   const std::string check = argv[1];
   if (check == "block_size_failure") block_size_failure();
   else if (check == "rest_hours") rest_hours();
   else if (check == "days_after_the_stop") days_after_the_stop();
   else if (check == "graphs_under_a_lockdown") graphs_under_a_lockdown();
+  else if (check == "small_handles_with_an_office_layout") small_handles_with_an_office_layout();
   else return 2;
   std::puts("ok");
 }

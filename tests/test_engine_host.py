@@ -21,7 +21,7 @@ def checks(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["block_size_failure", "rest_hours", "days_after_the_stop",
-                                   "graphs_under_a_lockdown"])
+                                   "graphs_under_a_lockdown", "small_handles_with_an_office_layout"])
 def test_engine(checks, check):
     out = subprocess.run([checks, check], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout + out.stderr
