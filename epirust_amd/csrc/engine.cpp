@@ -60,13 +60,15 @@ bool rect_inside(const Rect& r, uint32_t stride, uint32_t height) {
 }
 
 // A handle's device arrays: add() them, then alloc() them together. Below kOneAllocation bytes each
-// is an allocation of its own, which the runtime hands out from what it keeps (1M agents: created
-// in 0.85 ms and freed in 0.3, as one allocation 3.1 and 0.4); above, all are one, as freeing takes
-// its time per allocation (10M agents: freed in 3.3 ms, as one allocation 0.6; 32 runs of 100k 2.45,
-// 0.46; 64 of mixed sizes 3.3, 0.5; created in the same time). Larger arrays start on pages of
-// their own there too (10M agents 121.3 us an hour apart, 122.5 close together, 121.4 so).
+// is an allocation of its own, which the runtime hands out from what it keeps; above, all are one, as
+// freeing larger ones takes its time per allocation. Created and freed, apart and as one, where other
+// handles come between: 1M agents (61 MiB) 1.29 + 0.20 and 1.71 + 1.80 ms, 1.5M (95 MiB) 1.10 + 1.48
+// and 2.46 + 0.39, 1.7M (117 MiB) 1.22 + 1.98 and 2.30 + 0.43, 2M 1.18 + 2.19 and 1.67 + 0.37, 10M 2.27 + 3.10 and 2.39 + 0.39, 32 runs of
+// 100k 1.63 + 2.40 and 1.82 + 0.38; of one size after another as one is the quicker at all of these
+// sizes. Larger arrays start on pages of their own (10M agents 121.3 us an hour apart, 122.5 close
+// together, 121.4 so).
 struct DeviceBuffers {
-  static constexpr size_t kOneAllocation = 120u << 20, kPage = 2u << 20;
+  static constexpr size_t kOneAllocation = 100u << 20, kPage = 2u << 20;
   std::vector<void*> owned;
   std::vector<std::pair<void**, size_t>> arrays;  // added, not allocated yet: bytes
   template <class T>
