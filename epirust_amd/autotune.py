@@ -6,9 +6,10 @@ worker blocks pack whole offices into that many slots, so the second size also s
 many offices share a block's claim filter. For a workload (one or many simulation
 configs) the search is by coordinates: every home size with the office size equal to it,
 then every office size beside the best home size. Each candidate is timed over whole
-captured days on a fresh handle, the fastest pair is kept, and it is stored in tuning.json
-under a size class key derived from the simulation count and total agents, so later
-handles of the same class start with the tuned shape:
+captured days on fresh handles, and the fastest pair is kept, where an office size other than
+the home's has to gain more than the repeats of a candidate differ. It is stored in
+tuning.json under a size class key derived from the simulation count and total agents, so
+later handles of the same class start with the tuned shape:
 
     python -m epirust_amd.autotune tests/golden/configs/cfg4_replicates.json
 """
@@ -71,28 +72,31 @@ def _open(configs, seeds):
 
 
 def _time(configs, seeds, hours, repeats, block, office):
-    best = float("inf")
-    for _ in range(repeats):
+    """Seconds of each repeat, after an untimed one."""
+    times = []
+    for _ in range(repeats + 1):
         h = _open(configs, seeds)
         h.set_block_size(block)
         if office != block:
             h.set_office_block_size(office)
         t0 = time.perf_counter()
         h.step(hours)
-        best = min(best, time.perf_counter() - t0)
+        times.append(time.perf_counter() - t0)
         h.close()
-    return best
+    return times[1:]
 
 
 def tune(configs, seeds=None, hours=48, repeats=2, path=TUNING_PATH, candidates=CANDIDATES, verbose=True):
     """Time the candidate shapes on `hours` hours (whole days) and persist the best pair.
     Returns (home, office, {(home, office): seconds})."""
     seeds = seeds or [c.get("seed", 0) for c in configs]
-    results = {}
+    results, spread = {}, {}
 
     def run(block, office):
         if (block, office) not in results:
-            results[(block, office)] = _time(configs, seeds, hours, repeats, block, office)
+            times = _time(configs, seeds, hours, repeats, block, office)
+            results[(block, office)] = min(times)
+            spread[(block, office)] = max(times) - min(times)
             if verbose:
                 print("home %4d office %4d: %.3f ms per hour" % (block, office, 1e3 * results[(block, office)] / hours),
                       flush=True)
@@ -100,6 +104,8 @@ def tune(configs, seeds=None, hours=48, repeats=2, path=TUNING_PATH, candidates=
 
     block = min(candidates, key=lambda b: run(b, b))
     office = min(candidates, key=lambda o: run(block, o))
+    if results[(block, block)] - results[(block, office)] <= max(spread[(block, block)], spread[(block, office)]):
+        office = block
     table = load_table(path)
     table[size_class(configs)] = {
         "block": block, "office_block": office, "hours": hours,
@@ -116,7 +122,7 @@ def main(argv):
         with open(p) as f:
             cfg = json.load(f)
         configs = cfg if isinstance(cfg, list) else [cfg]
-        block, office, _ = tune(configs)
+        block, office, _ = tune(configs, hours=480, repeats=5)
         print("%s -> %s: home block %d, office block %d" % (p, size_class(configs), block, office))
 
 
