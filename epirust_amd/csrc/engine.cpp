@@ -198,7 +198,7 @@ struct epi_sim {
   uint32_t* pinned_active = nullptr;  // 2 x n_sims
   SimState* pinned_state = nullptr;   // n_sims: the states a step call reads back
   Counts7* pinned_rows = nullptr;     // n_rows: staging of the rows a step call returns
-  // the same three buffers' device addresses, which the export kernels write
+  // the same three buffers' device addresses, which kernels write
   uint32_t* d_pinned_active = nullptr;
   SimState* d_pinned_state = nullptr;
   Counts7* d_pinned_rows = nullptr;
@@ -657,7 +657,7 @@ int advance_streaming(epi_sim* s, uint32_t target) {
 }
 
 // Enqueue hours until `target` (or until every simulation has stopped). Whole days are
-// replayed from the captured graph; stop flags are polled one day behind the GPU.
+// replayed from captured graphs; the host polls the stop flags two graphs behind what it enqueues.
 int advance(epi_sim* s, uint32_t target) {
   s->last_loop_ms = 0.0;
   s->last_loop_hours = 0;

@@ -32,8 +32,8 @@
 //              block) claim nothing globally.
 //              Small handles, and days on which most agents are isolated, stay in the home
 //              layout throughout.
-//   k_night / k_quiet_hours: in day graphs, hours of day 1..6 (or 3..6) as one launch
-//              when no sweep can be pending inside them (no vaccination there).
+//   k_night / k_quiet_hours: hours of day 1..6 (or 3..6) of one call as one launch when no
+//              sweep can be pending inside them (no vaccination there).
 // A sweep decided at hour h (allocation_map.rs:306-337) is applied by the agent pass of
 // hour h+1 (before the routine, in k_step), which is what the reference's next hour sees;
 // sweeps are idempotent, so k_apply_sweep re-applies the last one before the host reads
@@ -457,8 +457,8 @@ __device__ __forceinline__ void add_event(const DevView& v, const EpiDesc& D, Si
 
 // What the epilogue reads besides the counts, loaded before the counts are reduced so the loads
 // overlap, by the whole block, so that it lies in scalar registers (thread 0's copy in vector
-// registers would set the register count of the whole commit): the simulation's descriptor and state, and the next entry
-// of the vaccination schedule.
+// registers would set the register count of the whole commit): the simulation's descriptor and
+// state, and the next entry of the vaccination schedule.
 struct EpilogueIn {
   EpiDesc D;
   SimState st;
@@ -822,14 +822,14 @@ __global__ void k_quiet_hours(DevView v, uint32_t n_hours) {
   if (threadIdx.x == 0) quiet_epilogues(v, blockIdx.x, n_hours);
 }
 
-// Hours of day 1..6 in one launch, for day graphs of simulations with no vaccination at
-// hours of day 1..5 (so the only sweep pending in the night is hour of day 0's). Blocks
+// Hours of day 1..6 in one launch, for days with no vaccination at hours of day 1..5 (so the only
+// sweep pending in the night is hour of day 0's) and no simulation's last hour at 1..6. Blocks
 // 0 .. n_epi-1 walk the six epilogues of simulation blockIdx.x; the agent blocks (home
 // layout) do the night's agent work: hour of day 0's sweep, every non-staff current area
 // to home (hour of day 1), and their share of the daily claim reset (hour of day 2). The
 // epilogues rewrite the parity slots meanwhile, so the agent blocks read hour of day 0's
 // sweep from its own slot, and whether the simulation runs from `active`, which these
-// hours cannot change (counts repeat, and a day graph never holds the last hour).
+// hours cannot change (counts repeat, and no simulation's hours end there).
 __global__ __attribute__((amdgpu_num_sgpr(80))) void k_night(DevView v, uint32_t n_epi) {
   if (blockIdx.x < n_epi) {  // uniform
     if (threadIdx.x == 0) quiet_epilogues(v, blockIdx.x, 6);

@@ -178,7 +178,7 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
 // ---- the network's stages
 
 // A block's LDS: MFMA operand fragments of 16 k (one row or column per half wave, 1 KiB each),
-// or a chunk of a bias gradient's rows. Two blocks fit a CU.
+// or a chunk of a bias gradient's rows. Four blocks' 38 KiB fit a CU's LDS.
 constexpr int kFrag = 512;  // bf16 values of a fragment
 constexpr int kArenaFrags = 38;
 

@@ -131,11 +131,11 @@ int epi_stream_citizen_states(epi_sim* sim, const char* path);
  * bytes) its length. No counterpart in the reference: a variant of the stream's device
  * formatter for callers that cannot allocate (code under HIP graph capture, serving loops,
  * harnesses that forbid hipMalloc). It calls no allocating routine: the formatter's
- * per-block offsets live in one static device array per GPU (512 KiB, held until the
- * process ends), so it handles at most 16,777,216 agents, and calls on one GPU that
- * overlap race on that array. cap must hold the records' upper bound, agents x the
- * longest record (EPI_ERR_ARG otherwise, before anything is launched). Single-simulation
- * handles only; returns once the text is written. */
+ * lengths, of each block of 256 agents' records and of each 16 blocks together, live in one
+ * static device array per GPU (512 KiB, held until the process ends), so it handles at most
+ * 16,777,216 agents, and calls on one GPU that overlap race on that array. cap must hold the
+ * records' upper bound, agents x the longest record (EPI_ERR_ARG otherwise, before anything
+ * is launched). Single-simulation handles only; returns once the text is written. */
 int epi_citizen_states_text_noalloc(epi_sim* sim, char* d_text, uint64_t cap, uint64_t* d_len);
 
 /* Counts of the last completed hour (hour 0: counts_at_start, engine/src/utils/util.rs:45-51). */
@@ -153,9 +153,9 @@ int epi_geometry(epi_sim* sim, uint32_t index, int32_t rects[20], uint32_t* hosp
 
 /* Profiling: runs n_hours with a HIP event pair around every kernel on the handle's stream
  * and returns the mean duration in ms of each of an hour's kernels (hospital scan; step;
- * the commit launch with its folded epilogue), each mean over the hours that launched it
- * (scan: hour of day 0; step: hours of day 0 and 7..23; commit: every hour), the number of
- * launches of each, and how many hours ran. */
+ * the commit launch with its folded epilogue, or the rest launch at hours of day 1..6), each
+ * mean over the hours that launched it (scan: hour of day 0; step: hours of day 0 and 7..23;
+ * commit: every hour), the number of launches of each, and how many hours ran. */
 int epi_profile(epi_sim* sim, uint32_t n_hours, double ms_mean[3], uint32_t launches[3], uint32_t* hours_run);
 
 /* Device time of the hour loop of the last epi_step / epi_batch_step / epi_run call: HIP
